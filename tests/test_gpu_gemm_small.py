@@ -1,0 +1,104 @@
+"""Small- and mid-M tiles of the bf16 GEMM (16 x 16 to 128 x 128 on the 16 x 16 x 32 MFMA): every
+row equals the row of a 256 x 256-tile call (32 x 32 x 16 MFMA) bit for bit, at sizes on both sides of
+each tile's limit, with partial last row tiles, at K values that leave out the deep-stage tiles, and with
+a row pitch too wide for 32-bit tile offsets."""
+
+import numpy as np
+import pytest
+import torch
+
+from yapd_amd import kernels
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+BIG = 16384
+
+
+def rnd(*shape, std=1.0, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return (torch.randn(*shape, generator=g, device="cuda") * std).to(BF)
+
+
+# N = 1024: 16 x 16 up to M = 128, 32 x 32 to 256, 64 x 32 to 512, 64 x 64 to 1024, 128 x 64 to 2048,
+# 128 x 128 to 4096
+SIZES = (1, 15, 17, 64, 128, 129, 256, 257, 511, 513, 1000, 1025, 1900, 2049, 3000, 4096)
+
+
+@pytest.mark.parametrize("epi", ["store", "residual"])
+@pytest.mark.parametrize("N,K", [(1024, 1024), (1024, 4096), (1000, 512)])
+def test_rows_equal_the_large_tiles(dev, epi, N, K):
+    A, W, R = rnd(BIG, K, std=0.5, seed=1), rnd(N, K, std=0.02, seed=2), rnd(BIG, N, seed=3)
+
+    def call(M):
+        C = R[:M].clone()
+        (kernels.gemm_bf16_residual if epi == "residual" else kernels.gemm_bf16)(A[:M], W, C)
+        return C
+
+    ref = call(BIG)
+    for M in SIZES:
+        assert torch.equal(call(M), ref[:M]), M
+
+
+@pytest.mark.parametrize("M", [1, 16, 33, 64, 100, 128, 200, 256, 300, 512, 900])
+def test_swiglu_rows_equal_the_large_tiles(dev, M):
+    A, W = rnd(8192, 1024, seed=4), rnd(8192, 1024, std=0.02, seed=5)
+    out = [torch.empty(m, 4096, dtype=BF, device=dev) for m in (8192, M)]
+    for o in out:
+        kernels.gemm_swiglu(A[: len(o)], W, o)
+    assert torch.equal(out[0][:M], out[1])
+
+
+@pytest.mark.parametrize("rows,bl", [(1, 1), (3, 5), (2, 32), (5, 32), (8, 16), (17, 13), (32, 16), (40, 32)])
+@pytest.mark.parametrize("H", [16, 4])
+def test_qkv_rows_equal_the_large_tiles(dev, rows, bl, H):
+    """Blocks that start at any slot of a page; H = 4: 64-column groups of q, k and v share a tile."""
+    D, big = 1024, 16384 // bl
+    A, W = rnd(big * bl, D, seed=6), rnd(3 * H * 64, D, std=0.02, seed=7)
+    fr = torch.outer(torch.arange(400.0), 10000.0 ** (-torch.arange(0, 64, 2) / 64))
+    cos, sin = (torch.cat([f, f], -1).to(BF).float().to(dev) for f in (fr.cos(), fr.sin()))
+    rng = np.random.default_rng(8)
+    pos0 = torch.from_numpy(rng.integers(0, 300, big).astype(np.int32)).to(dev)
+    cols = (300 + bl) // 16 + 1
+    table = torch.from_numpy(rng.permutation(big * cols).reshape(big, cols).astype(np.int32)).to(dev)
+    got = []
+    for n in (big, rows):
+        pool = torch.zeros(big * cols, 2, H, 1024, dtype=BF, device=dev)
+        q = torch.empty(n * bl, H * 64, dtype=BF, device=dev)
+        kernels.gemm_qkv_rope_kv(A[: n * bl], W, cos, sin, pos0[:n], bl, q, pool, table[:n])
+        got.append((q[: rows * bl], pool[table[:rows].long()]))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("rows,bl", [(1, 7), (2, 32), (9, 16), (30, 16), (70, 32)])
+def test_head_rows_equal_the_large_tiles(dev, rows, bl):
+    D, V, big = 1024, 8194, 8192 // bl
+    hid, ctx, W = rnd(big, bl, D, seed=9), rnd(big, 1, D, seed=10), rnd(V, D, std=0.02, seed=11)
+    out = [torch.empty(n, bl, 8200, dtype=BF, device=dev)[..., :V] for n in (big, rows)]
+    for o in out:
+        kernels.gemm_head_shift(hid[: len(o)], ctx[: len(o)], W, o)
+    assert torch.equal(out[0][:rows], out[1])
+
+
+@pytest.mark.parametrize("K", [64, 128, 192, 320, 1344])
+@pytest.mark.parametrize("M", [40, 1000, 3000])
+def test_short_and_odd_k(dev, K, M):
+    """Products of fp32 sums of K exact bf16 products against fp64, rounded to bf16: half a bf16 ulp
+    (2^-9 relative) plus the sums' own error, K * 2^-24 of the sum of magnitudes."""
+    A, W = rnd(M, K, seed=12), rnd(1024, K, std=0.02, seed=13)
+    C = torch.empty(M, 1024, dtype=BF, device=dev)
+    kernels.gemm_bf16(A, W, C)
+    ref = A.double() @ W.double().T
+    mag = A.double().abs() @ W.double().abs().T
+    assert ((C.double() - ref).abs() <= ref.abs() * 2.0 ** -8 + mag * K * 2.0 ** -24).all()
+
+
+def test_wide_row_pitch(dev):
+    """Rows further apart than 32-bit offsets in a tile reach: the same values as a packed call."""
+    M, N, K = 5, 64, 128
+    wide = torch.empty(M, (1 << 22) + 8, dtype=BF, device=dev)
+    A, W = rnd(M, K, seed=14), rnd(N, K, std=0.02, seed=15)
+    wide[:, :K] = A
+    out = [torch.empty(M, N, dtype=BF, device=dev) for _ in range(2)]
+    kernels.gemm_bf16(A, W, out[0])
+    kernels.gemm_bf16(wide[:, :K], W, out[1])
+    assert torch.equal(out[0], out[1])

@@ -2,19 +2,20 @@
 // row kernel.
 //
 // C[M, N] = A[M, K] * W[N, K]^T (nn.Linear layout), fp32 accumulation on
-// v_mfma_f32_32x32x16_bf16.  Grids of at least two 256 x 256 tiles per CU
-// (gate/up, QKV, the speech head), or one with the plain or residual epilogue
-// (o, down): `gemm_pt_kernel`, one persistent 4-wave workgroup per CU.  Other
-// large M: `gemm_dl_kernel`, a 256 x 256 tile of
-// 8 waves (128 x 64 each) whose A and W k-slices go global -> LDS by direct
-// loads into two 64 KB stages.  Small M: the same kernel on one-wave 64 x 64
-// tiles with three stages.  Mid M: the same kernel on 128 x 128 tiles of 8
-// waves (32 x 64 each).  `gemm_kernel` (register-staged tiles with padded LDS
-// rows) serves the quantised path below large M.  Every kernel runs the same MFMA over the same K
-// order, so a row's result does not depend on which kernel the batch size
-// selects.  Affine-quantised W: `gemm_dlq_kernel` (the direct-load layout with
-// W dequantised from registers into LDS) at large M, `gemm_kernel` below.  K
-// advances in steps of 64.
+// v_mfma_f32_32x32x16_bf16 or v_mfma_f32_16x16x32_bf16, whose sums over the same
+// K are equal bit for bit.  By the grid a tile size gives:
+//   * gemm_pt_kernel: 256 x 256 tiles, one persistent 4-wave workgroup per CU
+//     (at least two tiles per CU, one with the plain or residual epilogue);
+//   * gemm_dl_kernel: 256 x 256 tiles of 8 waves that fill three quarters of the
+//     CUs, and 128 x 128 tiles where those give more than one per CU;
+//   * gemm_sk_kernel: 16 x 16 to 128 x 128 tiles, the smallest with at most one
+//     workgroup per CU, as many LDS stages as fit (small and mid M).
+// A and W k-slices go global -> LDS by direct loads.  Affine-quantised W:
+// gemm_dlq_kernel (the direct-load layout with W dequantised from registers
+// into LDS) and, between its two tile sizes, gemm_kernel (register-staged tiles
+// with padded LDS rows).  Every kernel sums K in the same order, so a row's
+// result does not depend on which kernel the batch size selects.  K advances in
+// steps of 64.
 //
 // Epilogues (once per output element):
 //   * store    -- plain bf16 store (speech head, small projections);
@@ -33,6 +34,8 @@
 // A prologue mode "shift" reads A row (r, j) from hidden row (r, j-1) and
 // row (r, 0) from shift_ctx[r]: the token-shifted speech head
 // (engines/flashinfer.py:1452-1461).
+#include <type_traits>
+
 #include "common.h"
 #include "kv_layout.h"
 #include "packed.h"
@@ -59,7 +62,7 @@ struct Tile {
 constexpr int BK = 64;  // K granularity every config shares
 
 enum EpiMode { kEpiStore = 0, kEpiQkv = 1, kEpiSwiglu = 2, kEpiResidual = 3 };
-enum AMode { kAPlain = 0, kAShift = 1 };
+enum AMode { kAPlain = 0, kAShift = 1, kAWide = 2 };  // kAWide: plain, row pitches past 32-bit tile offsets
 
 struct GemmParams {
   const uint16_t* A;
@@ -173,6 +176,52 @@ __device__ __forceinline__ void stage_rope_rows(const GemmParams& p, const RowMe
   }
 }
 
+// One run of the qkv epilogue: dims d0 .. d0+3 (x0) and d0+32 .. d0+35 (x1) of
+// one head of token row m, its KV slot in `kv` (the head's K or V tile on the
+// token's page), cos/sin of the position at dims d0 .. d0+3.
+template <int SECTION>
+__device__ __forceinline__ void qkv_run(const GemmParams& p, const f32x4_t& x0, const f32x4_t& x1, const f32x4_t& c,
+                                        const f32x4_t& sn, uint16_t* kv, int slot, int m, int head, int d0) {
+  // Dims d0 + t (x0) and d0 + 32 + t (x1), rounded to bf16 two at a time:
+  // a packed pair holds dims (t, t + 1), which is also the store layout.
+  uint32_t X0[2], X1[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    X0[h] = pack_bf16x2(x0[2 * h], x0[2 * h + 1]);
+    X1[h] = pack_bf16x2(x1[2 * h], x1[2 * h + 1]);
+  }
+  if constexpr (SECTION < 2) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      // x*cos + rotate_half(x)*sin, rotate_half = [-x2, x1], each op rounded
+      // to bf16; bf16(-x2*s) = -bf16(x2*s) (round-to-nearest-even is symmetric)
+      const float a0 = bf16lo(X0[h]), a1 = bf16hi(X0[h]);
+      const float b0 = bf16lo(X1[h]), b1 = bf16hi(X1[h]);
+      const float c0 = c[2 * h], c1 = c[2 * h + 1], s0 = sn[2 * h], s1 = sn[2 * h + 1];
+      const uint32_t ac = pack_bf16x2(a0 * c0, a1 * c1), bs = pack_bf16x2(b0 * s0, b1 * s1);
+      const uint32_t bc = pack_bf16x2(b0 * c0, b1 * c1), as = pack_bf16x2(a0 * s0, a1 * s1);
+      X0[h] = pack_bf16x2(bf16lo(ac) - bf16lo(bs), bf16hi(ac) - bf16hi(bs));
+      X1[h] = pack_bf16x2(bf16lo(bc) + bf16lo(as), bf16hi(bc) + bf16hi(as));
+    }
+  }
+  const u32x2_t lo = {X0[0], X0[1]};
+  const u32x2_t hi = {X1[0], X1[1]};
+  if constexpr (SECTION == 0) {
+    uint16_t* qp = p.q_out + (static_cast<int64_t>(m) * p.n_heads + head) * kHeadDim + d0;
+    *reinterpret_cast<u32x2_t*>(qp) = lo;
+    *reinterpret_cast<u32x2_t*>(qp + 32) = hi;
+  } else if constexpr (SECTION == 1) {
+    *reinterpret_cast<u32x2_t*>(kv + slot * kHeadDim + d0) = lo;
+    *reinterpret_cast<u32x2_t*>(kv + slot * kHeadDim + d0 + 32) = hi;
+  } else {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      kv[(d0 + t) * kPageSize + slot] = static_cast<uint16_t>(X0[t >> 1] >> (16 * (t & 1)));
+      kv[(d0 + 32 + t) * kPageSize + slot] = static_cast<uint16_t>(X1[t >> 1] >> (16 * (t & 1)));
+    }
+  }
+}
+
 // qkv epilogue: NeoX RoPE on q and k from the cos/sin tables at each row's
 // position; the tables are HF's cat(freqs, freqs) layout, so column d + 32
 // equals column d and only columns 0..31 are read (staged in `rope`).  The qkv GEMM multiplies
@@ -204,46 +253,14 @@ __device__ __forceinline__ void epilogue_qkv_section(const GemmParams& p, const 
 #pragma unroll
     for (int r4 = 0; r4 < 4; ++r4) {
       const int d0 = 8 * r4 + dgrp;
-      // Dims d0 + t (x0) and d0 + 32 + t (x1), rounded to bf16 two at a time:
-      // a packed pair holds dims (t, t + 1), which is also the store layout.
-      uint32_t X0[2], X1[2];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        X0[h] = pack_bf16x2(acc[i][2 * q2][4 * r4 + 2 * h], acc[i][2 * q2][4 * r4 + 2 * h + 1]);
-        X1[h] = pack_bf16x2(acc[i][2 * q2 + 1][4 * r4 + 2 * h], acc[i][2 * q2 + 1][4 * r4 + 2 * h + 1]);
-      }
+      const f32x16_t &x0 = acc[i][2 * q2], &x1 = acc[i][2 * q2 + 1];
+      f32x4_t c{}, sn{};
       if constexpr (SECTION < 2) {
-        const f32x4_t c = *reinterpret_cast<const f32x4_t*>(rope + rl * kRopePitch + d0);
-        const f32x4_t sn = *reinterpret_cast<const f32x4_t*>(rope + (T::BM + rl) * kRopePitch + d0);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          // x*cos + rotate_half(x)*sin, rotate_half = [-x2, x1], each op rounded
-          // to bf16; bf16(-x2*s) = -bf16(x2*s) (round-to-nearest-even is symmetric)
-          const float a0 = bf16lo(X0[h]), a1 = bf16hi(X0[h]);
-          const float b0 = bf16lo(X1[h]), b1 = bf16hi(X1[h]);
-          const float c0 = c[2 * h], c1 = c[2 * h + 1], s0 = sn[2 * h], s1 = sn[2 * h + 1];
-          const uint32_t ac = pack_bf16x2(a0 * c0, a1 * c1), bs = pack_bf16x2(b0 * s0, b1 * s1);
-          const uint32_t bc = pack_bf16x2(b0 * c0, b1 * c1), as = pack_bf16x2(a0 * s0, a1 * s1);
-          X0[h] = pack_bf16x2(bf16lo(ac) - bf16lo(bs), bf16hi(ac) - bf16hi(bs));
-          X1[h] = pack_bf16x2(bf16lo(bc) + bf16lo(as), bf16hi(bc) + bf16hi(as));
-        }
+        c = *reinterpret_cast<const f32x4_t*>(rope + rl * kRopePitch + d0);
+        sn = *reinterpret_cast<const f32x4_t*>(rope + (T::BM + rl) * kRopePitch + d0);
       }
-      const u32x2_t lo = {X0[0], X0[1]};
-      const u32x2_t hi = {X1[0], X1[1]};
-      if constexpr (SECTION == 0) {
-        uint16_t* qp = p.q_out + static_cast<int64_t>(m) * HD + head * kHeadDim + d0;
-        *reinterpret_cast<u32x2_t*>(qp) = lo;
-        *reinterpret_cast<u32x2_t*>(qp + 32) = hi;
-      } else if constexpr (SECTION == 1) {
-        *reinterpret_cast<u32x2_t*>(kv + slot * kHeadDim + d0) = lo;
-        *reinterpret_cast<u32x2_t*>(kv + slot * kHeadDim + d0 + 32) = hi;
-      } else {
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          kv[(d0 + t) * kPageSize + slot] = static_cast<uint16_t>(X0[t >> 1] >> (16 * (t & 1)));
-          kv[(d0 + 32 + t) * kPageSize + slot] = static_cast<uint16_t>(X1[t >> 1] >> (16 * (t & 1)));
-        }
-      }
+      qkv_run<SECTION>(p, f32x4_t{x0[4 * r4], x0[4 * r4 + 1], x0[4 * r4 + 2], x0[4 * r4 + 3]},
+                       f32x4_t{x1[4 * r4], x1[4 * r4 + 1], x1[4 * r4 + 2], x1[4 * r4 + 3]}, c, sn, kv, slot, m, head, d0);
     }
   }
 }
@@ -270,6 +287,16 @@ __device__ __forceinline__ void epilogue_qkv(const GemmParams& p, const f32x16_t
   }
 }
 
+// silu(g) * u of two neighbouring features, rounded as the reference's separate
+// ops are, packed.
+__device__ __forceinline__ uint32_t silu_mul(float g0, float g1, float u0, float u1) {
+  const uint32_t gp = pack_bf16x2(g0, g1), up = pack_bf16x2(u0, u1);
+  const float gb0 = bf16lo(gp), gb1 = bf16hi(gp);
+  const uint32_t sp = pack_bf16x2(gb0 * __builtin_amdgcn_rcpf(1.f + __expf(-gb0)),
+                                  gb1 * __builtin_amdgcn_rcpf(1.f + __expf(-gb1)));
+  return pack_bf16x2(bf16lo(sp) * bf16lo(up), bf16hi(sp) * bf16hi(up));
+}
+
 // swiglu epilogue.  Each 64-column group of W holds the gate rows of 32
 // features, then their up rows, so tiles 2q and 2q+1 of a wave are gate and
 // up of the same 32 features.  The swiglu GEMM multiplies W x A^T (MFMA
@@ -287,13 +314,6 @@ __device__ __forceinline__ void epilogue_swiglu(const GemmParams& p, const f32x1
   const int tok = lane & 31;
   const int fsub = 4 * (lane >> 5);
   const bool vec_ok = (p.ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(p.C) & 7u) == 0);
-  auto silu_mul = [](float g0, float g1, float u0, float u1) {
-    const uint32_t gp = pack_bf16x2(g0, g1), up = pack_bf16x2(u0, u1);
-    const float gb0 = bf16lo(gp), gb1 = bf16hi(gp);
-    const uint32_t sp = pack_bf16x2(gb0 * __builtin_amdgcn_rcpf(1.f + __expf(-gb0)),
-                                    gb1 * __builtin_amdgcn_rcpf(1.f + __expf(-gb1)));
-    return pack_bf16x2(bf16lo(sp) * bf16lo(up), bf16hi(sp) * bf16hi(up));
-  };
 #pragma unroll
   for (int i = 0; i < T::TM; ++i) {
     const int m = m0 + wm * T::WTM + 32 * i + tok;
@@ -647,11 +667,10 @@ __global__ __launch_bounds__(T::THREADS) void gemm_kernel(const GemmParams p) {
 // bank groups (two 128-byte rows share one 256-byte bank line).  A load
 // instruction covers 8 rows; lane i writes slot i % 8 of row i / 8, so it
 // fetches the chunk that belongs there.
-template <class T, int NS>
+template <class T>
 struct DlLayout {
   static_assert(T::BK == 64, "direct-load tiles use 128-byte LDS rows");
   static constexpr int WAVES = T::THREADS / 64;
-  static_assert(NS >= 2 && NS <= 4, "two to four LDS stages");
   static constexpr int ROWB = 128;
   static constexpr int CPR = 8;  // 16-byte chunks per row
   static constexpr int RPI = 8;  // rows per 1 KB load instruction
@@ -661,27 +680,15 @@ struct DlLayout {
   static constexpr int LA = T::BM / 8 / WAVES;  // 1 KB loads per wave and k-tile
   static constexpr int LB = T::BN / 8 / WAVES;
   static_assert(LA * 8 * WAVES == T::BM && LB * 8 * WAVES == T::BN, "rows must split evenly over the waves");
-  static constexpr int LPT = LA + LB;  // loads per wave and k-tile
-  static_assert((NS - 2) * LPT <= 63, "the vmcnt counter holds at most 63 loads");
   static constexpr int C_BYTES = T::BM * (T::BN + 8) * 2;  // store-epilogue staging
-  static constexpr int LDS = NS * STAGE > C_BYTES ? NS * STAGE : C_BYTES;
+  static constexpr int LDS = 2 * STAGE > C_BYTES ? 2 * STAGE : C_BYTES;
 };
 
-// Wait until at most N of this wave's vector-memory loads are outstanding
-// (they complete in issue order).  The memory clobber keeps the LDS reads
-// that follow below the wait.
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-// Hand-off of an LDS stage across the workgroup: this wave's loads up to the
-// stage have landed (at most N later loads still in flight), its LDS reads
-// have completed (so the stage it read last may be overwritten), then the
-// workgroup barrier.  __syncthreads would also drain the later tiles' loads.
-template <int N>
+// Hand-off of an LDS stage across the workgroup: this wave's loads have landed
+// and its LDS reads have completed (so the stage it read last may be
+// overwritten), then the workgroup barrier.
 __device__ __forceinline__ void stage_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
 // 16 bytes per lane from src into LDS at lds_run + 16 * lane (lds_run must be
@@ -691,9 +698,25 @@ __device__ __forceinline__ void load_lds16(const uint16_t* src, char* lds_run) {
       src, reinterpret_cast<__attribute__((address_space(3))) void*>(reinterpret_cast<uintptr_t>(lds_run)), 16, 0, 0);
 }
 
-template <class T, int EPI, int AM, int NS>
+// The same through a buffer descriptor: bytes [ofs + sofs, +16) per lane from
+// the descriptor's base (ofs per lane, sofs uniform).  A buffer load is no FLAT
+// instruction, so the compiler's waits for LDS reads stay counted ones; with
+// global_load_lds in flight it waits for every LDS read outstanding
+// (lgkmcnt(0)) before each use of a fragment.
+__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t rsrc, uint32_t ofs, uint32_t sofs, char* lds_run) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(
+      rsrc, reinterpret_cast<__attribute__((address_space(3))) void*>(reinterpret_cast<uintptr_t>(lds_run)), 16, ofs,
+      sofs, 0, 0);
+}
+
+// Descriptor over the 4 GiB from p on (word 3: raw 32-bit elements, no swizzle).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_from(const uint16_t* p) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p), 0, -1, 0x00020000);
+}
+
+template <class T, int EPI, int AM>
 __global__ __launch_bounds__(T::THREADS) void gemm_dl_kernel(const GemmParams p) {
-  using L = DlLayout<T, NS>;
+  using L = DlLayout<T>;
   // Dynamic LDS: the compiler cannot see the DMA writes into a static
   // __shared__ array and would treat its contents as undefined.
   extern __shared__ __attribute__((aligned(16))) uint16_t dyn_lds[];
@@ -706,28 +729,53 @@ __global__ __launch_bounds__(T::THREADS) void gemm_dl_kernel(const GemmParams p)
 
   // Per-lane sources of this wave's LA + LB loads (k offset added per tile).
   // Rows past M (N) re-read the last valid row, as in the staged kernel.
+  // Plain A: buffer descriptors from the tile's first rows on, 32-bit offsets.
+  constexpr bool kBuf = AM == kAPlain;
+  const __amdgpu_buffer_rsrc_t ra = buffer_from(p.A + static_cast<int64_t>(m0) * p.lda);
+  const __amdgpu_buffer_rsrc_t rw = buffer_from(p.W + static_cast<int64_t>(n0) * p.ldw);
   const uint16_t* a_src[L::LA];
   const uint16_t* b_src[L::LB];
+  uint32_t a_ofs[L::LA], b_ofs[L::LB];
 #pragma unroll
   for (int j = 0; j < L::LA; ++j) {
     const int r = (wave * L::LA + j) * 8 + (lane >> 3);
     const int c = (lane & 7) ^ ((r >> 1) & 7);
-    a_src[j] = a_row_ptr<AM>(p, min(m0 + r, p.M - 1)) + 8 * c;
+    if constexpr (kBuf) {
+      a_ofs[j] = static_cast<uint32_t>((static_cast<int64_t>(min(r, p.M - 1 - m0)) * p.lda + 8 * c) * 2);
+    } else {
+      a_src[j] = a_row_ptr<AM>(p, min(m0 + r, p.M - 1)) + 8 * c;
+    }
   }
 #pragma unroll
   for (int j = 0; j < L::LB; ++j) {
     const int r = (wave * L::LB + j) * 8 + (lane >> 3);
     const int c = (lane & 7) ^ ((r >> 1) & 7);
-    b_src[j] = p.W + static_cast<int64_t>(min(n0 + r, p.N - 1)) * p.ldw + 8 * c;
+    if constexpr (kBuf) {
+      b_ofs[j] = static_cast<uint32_t>((static_cast<int64_t>(min(r, p.N - 1 - n0)) * p.ldw + 8 * c) * 2);
+    } else {
+      b_src[j] = p.W + static_cast<int64_t>(min(n0 + r, p.N - 1)) * p.ldw + 8 * c;
+    }
   }
   auto issue = [&](int kt, int stage) {
     const int k = kt * T::BK;
     char* a_dst = lds + stage * L::STAGE + wave * L::LA * 1024;
     char* b_dst = lds + stage * L::STAGE + L::A_BYTES + wave * L::LB * 1024;
 #pragma unroll
-    for (int j = 0; j < L::LA; ++j) load_lds16(a_src[j] + k, a_dst + j * 1024);
+    for (int j = 0; j < L::LA; ++j) {
+      if constexpr (kBuf) {
+        load_lds16(ra, a_ofs[j], 2 * k, a_dst + j * 1024);
+      } else {
+        load_lds16(a_src[j] + k, a_dst + j * 1024);
+      }
+    }
 #pragma unroll
-    for (int j = 0; j < L::LB; ++j) load_lds16(b_src[j] + k, b_dst + j * 1024);
+    for (int j = 0; j < L::LB; ++j) {
+      if constexpr (kBuf) {
+        load_lds16(rw, b_ofs[j], 2 * k, b_dst + j * 1024);
+      } else {
+        load_lds16(b_src[j] + k, b_dst + j * 1024);
+      }
+    }
   };
 
   f32x16_t acc[T::TM][T::TN];
@@ -782,69 +830,327 @@ __global__ __launch_bounds__(T::THREADS) void gemm_dl_kernel(const GemmParams p)
     __builtin_amdgcn_sched_group_barrier(0x008, T::TM * T::TN - (T::TM + T::TN), 0);
   };
 
-  // NS LDS stages, NS - 1 tiles in flight.  Tile kt+NS-1 is requested at the
-  // top of tile kt into the stage tile kt-1 used: its last fragments were
-  // consumed by the MFMAs that ended tile kt-1.  Before the first fragments
-  // of tile kt+1 are read, the wave waits for its loads of that tile and
-  // keeps the later tiles in flight; with several waves a barrier then covers
-  // the other waves' loads of it (with two stages nothing later is in flight
-  // and __syncthreads does both).
+  // Two LDS stages: tile kt + 1 is requested at the top of tile kt into the stage
+  // tile kt - 1 used (its last fragments were consumed by the MFMAs that ended
+  // it); the barrier before its first fragments are read waits for its loads.
   const int kt_n = p.K / T::BK;
-#pragma unroll
-  for (int s = 0; s + 1 < NS; ++s)
-    if (s < kt_n) issue(s, s);
+  issue(0, 0);
   const RowMeta rm = EPI == kEpiQkv ? qkv_row_meta<T>(p, m0, tid) : RowMeta{0, 0};
-  // Tiles issued after tile t, when the fragments of tile t are first read.
-  auto wait_tile = [&](int t) {
-    if constexpr (NS == 2) {
-      if constexpr (L::WAVES > 1) {
-        __syncthreads();
-      } else {
-        wait_vmcnt<0>();
-      }
-    } else {
-      // the same condition in every wave: all of them take the same barriers
-      const bool full = min(t + NS - 2, kt_n - 1) - t == NS - 2;
-      if constexpr (L::WAVES > 1) {
-        if (full) {
-          stage_barrier<(NS - 2) * L::LPT>();
-        } else {
-          stage_barrier<0>();
-        }
-      } else {
-        if (full) {
-          wait_vmcnt<(NS - 2) * L::LPT>();
-        } else {
-          wait_vmcnt<0>();
-        }
-      }
-    }
-  };
-  wait_tile(0);
+  stage_barrier();
   read_frags(0, 0, 0);
-  int stage = 0;
   for (int kt = 0; kt < kt_n; ++kt) {
+    const int stage = kt & 1;
     const bool more = kt + 1 < kt_n;
-    const int next = stage + 1 == NS ? 0 : stage + 1;
-    if (kt + NS - 1 < kt_n) issue(kt + NS - 1, stage == 0 ? NS - 1 : stage - 1);
+    if (more) issue(kt + 1, stage ^ 1);
 #pragma unroll
     for (int ks = 0; ks + 1 < KS; ++ks) {
       read_frags(stage, ks + 1, (ks + 1) & 1);
       mfma_step(ks & 1);
       interleave();
     }
-    if (more) {
-      wait_tile(kt + 1);
-      read_frags(next, 0, 0);
-    } else if constexpr (L::WAVES > 1) {
-      __syncthreads();  // every wave is done with the stages before the epilogue reuses LDS
-    }
+    // after the last tile: every wave is done with the stages before the epilogue reuses LDS
+    stage_barrier();
+    if (more) read_frags(stage ^ 1, 0, 0);
     mfma_step((KS - 1) & 1);
     if (more) interleave();
-    stage = next;
   }
   static_assert(EPI != kEpiQkv || qkv_lds_bytes<T>() <= L::LDS, "qkv epilogue LDS");
   finish_tile<T, EPI>(p, acc, dyn_lds, rm, m0, n0, wm, wn, lane, tid);
+}
+
+// ---------------------------------------------------------------------------
+// Small and mid M: tiles of 16 x 16 sub-tiles (v_mfma_f32_16x16x32_bf16).
+//
+// At few rows the weights' bytes bound the product (8 MB for down: ~1.7 us), but
+// a CU fills its LDS at no more than 64 B/clk with ~1 us of latency, so what
+// counts is every CU loading with up to 144 KB in flight: small tiles, deep
+// stages, no more bytes per CU than needed.  WM x WN compute waves own TM x TN
+// sub-tiles each; all WAVES waves load.  A stage holds S k-tiles of 64: per
+// k-tile the BM rows of A, then the BN rows of W, 128 bytes a row, swizzled as
+// in gemm_dl_kernel.  The 16 x 16 MFMA keeps the serial chain of one tile short
+// (K = 4096: 128 MFMAs of 16 clk against 256 of 32).  The product is transposed
+// (W x A^T): a lane holds one token and runs of 4 consecutive columns, stored
+// from registers.  For the paired epilogues a wave's sub-tiles 2q and 2q + 1
+// are 16 columns and the 16 columns 32 further on (RoPE's dims d and d + 32;
+// gate and up of one feature).
+//
+// down, M = 64 (us): one-wave 64 x 64 tiles, three stages 33.8; 16 x 16 tiles
+// with every wait for LDS at lgkmcnt(0) 10.2; counted waits (buffer loads) 6.0.
+template <int TM_, int TN_, int WM_, int WN_, int WAVES_, int S_, int NS_, int P_>
+struct SkTile {
+  static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, WAVES = WAVES_, S = S_, NS = NS_, P = P_;
+  static constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
+  static constexpr int THREADS = 64 * WAVES;
+  static constexpr int RG = (BM + BN) / 8;  // 1 KB loads per k-tile
+  static constexpr int PW = RG / WAVES;     // of them per wave
+  static constexpr int LPS = PW * S;        // loads per wave and stage
+  static constexpr int KT = RG * 1024;      // bytes of one k-tile
+  static constexpr int STAGE = S * KT;
+  static constexpr int LDS = NS * STAGE;
+  static_assert(PW * WAVES == RG && WM * WN <= WAVES, "loads must split evenly over the waves");
+  static_assert((NS - 2) * LPS <= 63 && LDS <= 160 * 1024 && NS >= 3, "vmcnt / LDS limits");
+  static_assert((2 * S) % P == 0, "fragment slots must cycle with the stage");
+};
+
+// Wait until at most N of this wave's loads are in flight, then the workgroup barrier.
+template <int N>
+__device__ __forceinline__ void wait_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+// wait_barrier<later * LPT> for a `later` <= MAX that is the same in every wave.
+template <int MAX, int LPT>
+__device__ __forceinline__ void wait_barrier_later(int later) {
+  if constexpr (MAX == 0) {
+    wait_barrier<0>();
+  } else {
+    if (later >= MAX) {
+      wait_barrier<MAX * LPT>();
+    } else {
+      wait_barrier_later<MAX - 1, LPT>(later);
+    }
+  }
+}
+
+template <class T, int EPI, int AM>
+__global__ __launch_bounds__(T::THREADS) void gemm_sk_kernel(const GemmParams p) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t dyn_lds[];
+  char* lds = reinterpret_cast<char*>(dyn_lds);
+  constexpr bool kPair = EPI == kEpiQkv || EPI == kEpiSwiglu;
+  static_assert(!kPair || T::TN % 2 == 0, "pair epilogues need both halves in a wave");
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wm = wave / T::WN, wn = wave % T::WN;
+  // Workgroup L runs on XCD L % 8: each XCD takes a contiguous run of tiles, in
+  // row bands (columns fastest) with xcd_band, else column bands (rows fastest).
+  int bx, by;
+  {
+    const int C = gridDim.x, R = gridDim.y, n = C * R;
+    const int L = blockIdx.x + C * blockIdx.y;
+    const int x = L % 8;
+    const int t = x * (n / 8) + min(x, n % 8) + L / 8;
+    by = p.xcd_band ? t / C : t % R;
+    bx = p.xcd_band ? t % C : t / R;
+  }
+  const int m0 = by * T::BM;
+  // W row of local column b
+  auto w_col = [&](int b) {
+    if constexpr (kPair) {
+      const int u = bx * (T::BN / 32) + (b >> 5), w = b & 31;
+      return 64 * (u >> 1) + 16 * (u & 1) + (w < 16 ? w : w + 16);
+    } else {
+      return bx * T::BN + b;
+    }
+  };
+  const int kt_n = p.K / 64;
+  const int st_n = kt_n / T::S;
+  // Loads: row groups of 8 rows, T::PW of them per wave.  Through buffer
+  // descriptors from the tile's first row of A and of W on, except for the
+  // shifted A, whose rows come from two arrays.
+  constexpr bool kBuf = AM == kAPlain;
+  const int w0 = kPair ? bx * T::BN & ~63 : bx * T::BN;  // first W row
+  const __amdgpu_buffer_rsrc_t ra = buffer_from(p.A + static_cast<int64_t>(m0) * p.lda);
+  const __amdgpu_buffer_rsrc_t rw = buffer_from(p.W + static_cast<int64_t>(w0) * p.ldw);
+  const uint16_t* src[T::PW];
+  uint32_t ofs[T::PW];
+#pragma unroll
+  for (int j = 0; j < T::PW; ++j) {
+    const int r = (wave * T::PW + j) * 8 + (lane >> 3);
+    const int c = (lane & 7) ^ ((r >> 1) & 7);
+    const bool is_a = (wave * T::PW + j) * 8 < T::BM;
+    if constexpr (kBuf) {
+      const int64_t e = is_a ? static_cast<int64_t>(min(r, p.M - 1 - m0)) * p.lda
+                             : static_cast<int64_t>(min(w_col(r - T::BM), p.N - 1) - w0) * p.ldw;
+      ofs[j] = static_cast<uint32_t>((e + 8 * c) * 2);
+    } else {
+      src[j] = (is_a ? a_row_ptr<AM>(p, min(m0 + r, p.M - 1))
+                     : p.W + static_cast<int64_t>(min(w_col(r - T::BM), p.N - 1)) * p.ldw) + 8 * c;
+    }
+  }
+  auto issue = [&](int st, int slot) {
+    char* dst = lds + slot * T::STAGE + wave * T::PW * 1024;
+#pragma unroll
+    for (int s = 0; s < T::S; ++s) {
+      const int k = (st * T::S + s) * 64;
+#pragma unroll
+      for (int j = 0; j < T::PW; ++j) {
+        if constexpr (kBuf) {
+          load_lds16((wave * T::PW + j) * 8 < T::BM ? ra : rw, ofs[j], 2 * k, dst + s * T::KT + j * 1024);
+        } else {
+          load_lds16(src[j] + k, dst + s * T::KT + j * 1024);
+        }
+      }
+    }
+  };
+  const int tok = lane & 15, sub = 4 * (lane >> 4);
+  // token rows of this lane
+  int pos[T::TM];
+  int prow[T::TM];
+  if constexpr (EPI == kEpiQkv) {
+#pragma unroll
+    for (int i = 0; i < T::TM; ++i) {
+      const int m = min(m0 + (wm * T::TM + i) * 16 + tok, p.M - 1);
+      int r, slot;
+      if (p.tok_row != nullptr) {
+        r = min(max(p.tok_row[m], 0), p.n_rows - 1);
+        slot = m - p.row_start[r];
+      } else {
+        r = m / p.bl;
+        slot = m - r * p.bl;
+      }
+      prow[i] = r;
+      pos[i] = p.pos0[r] + slot;
+    }
+  }
+#pragma unroll
+  for (int s = 0; s + 1 < T::NS; ++s)
+    if (s < st_n) issue(s, s);
+
+  f32x4_t acc[T::TM][T::TN];
+#pragma unroll
+  for (int i = 0; i < T::TM; ++i)
+#pragma unroll
+    for (int j = 0; j < T::TN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int sw = (tok >> 1) & 7, cg = lane >> 4;
+  const int a_off = (wm * T::TM * 16 + tok) * 128;
+  const int b_off = (T::BM + wn * T::TN * 16 + tok) * 128;
+  // Fragments are read P k-steps (of 32) ahead of their MFMAs, across stages:
+  // the barrier that hands stage st + 1 over stands P k-steps before the end of
+  // stage st.  Behind it stage st + NS - 1 is requested into the slot of stage
+  // st - 1, whose fragments every wave had consumed when it reached the barrier.
+  constexpr int N = 2 * T::S, P = T::P;
+  bf16x8_t a[P][T::TM], b[P][T::TN];
+  auto read = [&](const char* base, int ks, int q) {
+    const int co = ((4 * (ks & 1) + cg) ^ sw) * 16 + (ks >> 1) * T::KT;
+#pragma unroll
+    for (int j = 0; j < T::TN; ++j) b[q][j] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(base + b_off + j * 2048 + co));
+#pragma unroll
+    for (int i = 0; i < T::TM; ++i) a[q][i] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(base + a_off + i * 2048 + co));
+  };
+  // Hand stage st + 1 over and request stage st + NS - 1 (while there is one).
+  auto hand_over = [&](int st, int slot, auto steady) {
+    if constexpr (decltype(steady)::value) {
+      wait_barrier<(T::NS - 3) * T::LPS>();
+      issue(st + T::NS - 1, slot == 0 ? T::NS - 1 : slot - 1);
+    } else {
+      wait_barrier_later<T::NS - 3, T::LPS>(min(T::NS - 3, st_n - 2 - st));
+    }
+  };
+  wait_barrier_later<T::NS - 2, T::LPS>(min(T::NS - 2, st_n - 1));
+  int slot = 0, st = 0;
+  const auto advance = [&]() { slot = slot + 1 == T::NS ? 0 : slot + 1; };
+  if (wave >= T::WM * T::WN) {  // waves that only load
+    for (; st + T::NS - 1 < st_n; ++st, advance()) hand_over(st, slot, std::true_type{});
+    for (; st + 1 < st_n; ++st) hand_over(st, slot, std::false_type{});
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < P; ++q) read(lds, q, q);
+  // MODE 0: stages follow and loads go out; 1: stages follow; 2: the last stage
+  auto stage = [&](auto mode) {
+    constexpr int MODE = decltype(mode)::value;
+    const char* base = lds + slot * T::STAGE;
+    const char* nbase = lds + (slot + 1 == T::NS ? 0 : slot + 1) * T::STAGE;
+#pragma unroll
+    for (int ks = 0; ks < N; ++ks) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < T::TM; ++i)
+#pragma unroll
+        for (int j = 0; j < T::TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[ks % P][j], a[ks % P][i], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (MODE < 2) {
+        if (ks + P == N) hand_over(st, slot, std::bool_constant<MODE == 0>{});
+      }
+      if (ks + P < N) {
+        read(base, ks + P, ks % P);
+      } else if constexpr (MODE < 2) {
+        read(nbase, ks + P - N, ks % P);
+      }
+    }
+    advance();
+    ++st;
+  };
+  while (st + T::NS - 1 < st_n) stage(std::integral_constant<int, 0>{});
+  while (st + 1 < st_n) stage(std::integral_constant<int, 1>{});
+  stage(std::integral_constant<int, 2>{});
+#pragma unroll
+  for (int i = 0; i < T::TM; ++i) {
+    const int m = m0 + (wm * T::TM + i) * 16 + tok;
+    if (m >= p.M) continue;
+    if constexpr (!kPair) {
+      const bool vec_ok = (p.ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(p.C) & 7u) == 0);
+      uint16_t* const row = p.C + static_cast<int64_t>(m) * p.ldc;
+#pragma unroll
+      for (int j = 0; j < T::TN; ++j) {
+        const int n = bx * T::BN + (wn * T::TN + j) * 16 + sub;
+        u32x2_t v = {pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3])};
+        if (vec_ok && n + 4 <= p.N) {
+          if constexpr (EPI == kEpiResidual) {
+            const u32x2_t r = *reinterpret_cast<const u32x2_t*>(row + n);
+#pragma unroll
+            for (int w = 0; w < 2; ++w)
+              v[w] = pack_bf16x2(bf16lo(r[w]) + bf16lo(v[w]), bf16hi(r[w]) + bf16hi(v[w]));
+          }
+          *reinterpret_cast<u32x2_t*>(row + n) = v;
+        } else {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            if (n + t >= p.N) break;
+            const uint32_t x = (v[t >> 1] >> (16 * (t & 1))) & 0xffffu;
+            row[n + t] = static_cast<uint16_t>(
+                EPI == kEpiResidual ? f32_to_bf16(bf16_to_f32(row[n + t]) + bf16_to_f32(x)) : x);
+          }
+        }
+      }
+    } else if constexpr (EPI == kEpiSwiglu) {
+      const bool vec_ok = (p.ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(p.C) & 7u) == 0);
+      uint16_t* const row = p.C + static_cast<int64_t>(m) * p.ldc;
+#pragma unroll
+      for (int j = 0; j < T::TN; j += 2) {
+        const int u = bx * (T::BN / 32) + (wn * T::TN + j) / 2;
+        if (32 * u >= p.N) continue;
+        const f32x4_t &g = acc[i][j], &h = acc[i][j + 1];
+        const u32x2_t y = {silu_mul(g[0], g[1], h[0], h[1]), silu_mul(g[2], g[3], h[2], h[3])};
+        uint16_t* dst = row + 16 * u + sub;
+        if (vec_ok) {
+          *reinterpret_cast<u32x2_t*>(dst) = y;
+        } else {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) dst[t] = static_cast<uint16_t>(y[t >> 1] >> (16 * (t & 1)));
+        }
+      }
+    } else {
+      const int HD = p.n_heads * kHeadDim;
+      const int pi = min(max(pos[i], 0) / kPageSize, p.table_cols - 1);
+      int64_t page = p.table[static_cast<int64_t>(prow[i]) * p.table_stride + pi];
+      page = min(max(page, int64_t{0}), p.n_pages - 1);
+      const int pc = min(max(pos[i], 0), p.max_pos - 1);
+#pragma unroll
+      for (int j = 0; j < T::TN; j += 2) {
+        const int u = bx * (T::BN / 32) + (wn * T::TN + j) / 2;
+        const int nb = 64 * (u >> 1);
+        if (nb >= p.N) continue;
+        const int section = nb / HD;
+        const int head = (nb - section * HD) / kHeadDim;
+        const int d0 = 16 * (u & 1) + sub;
+        uint16_t* const kv = p.pool + kv_plane_offset(page, section == 2 ? 1 : 0, head, p.n_heads);
+        if (section < 2) {
+          const f32x4_t c = *reinterpret_cast<const f32x4_t*>(p.cos_t + pc * kHeadDim + d0);
+          const f32x4_t sn = *reinterpret_cast<const f32x4_t*>(p.sin_t + pc * kHeadDim + d0);
+          if (section == 0) {
+            qkv_run<0>(p, acc[i][j], acc[i][j + 1], c, sn, kv, pos[i] & (kPageSize - 1), m, head, d0);
+          } else {
+            qkv_run<1>(p, acc[i][j], acc[i][j + 1], c, sn, kv, pos[i] & (kPageSize - 1), m, head, d0);
+          }
+        } else {
+          const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+          qkv_run<2>(p, acc[i][j], acc[i][j + 1], z, z, kv, pos[i] & (kPageSize - 1), m, head, d0);
+        }
+      }
+    }
+  }
 }
 
 // Affine-quantised W on the direct-load layout: A moves global -> LDS by
@@ -860,7 +1166,7 @@ __global__ __launch_bounds__(T::THREADS) void gemm_dl_kernel(const GemmParams p)
 // the dequantised weights bit for bit (same W values, MFMA and K order).
 template <class T, int EPI, int AM, int BQ>
 __global__ __launch_bounds__(T::THREADS) void gemm_dlq_kernel(const GemmParams p) {
-  using L = DlLayout<T, 2>;
+  using L = DlLayout<T>;
   static_assert(BQ == 4 || BQ == 8, "4- or 8-bit codes");
   extern __shared__ __attribute__((aligned(16))) uint16_t dyn_lds[];
   char* lds = reinterpret_cast<char*>(dyn_lds);
@@ -1487,23 +1793,23 @@ int launch_tile(const GemmParams& p, hipStream_t st) {
   return YAPD_OK;
 }
 
-template <class T, int EPI, int AM, int NS = 2>
+template <class T, int EPI, int AM>
 int launch_dl(const GemmParams& p, hipStream_t st) {
-  using L = DlLayout<T, NS>;
+  using L = DlLayout<T>;
   // The dynamic-LDS limit is raised once per kernel and device (setting it
   // twice, e.g. from two threads, is harmless).
   static bool lds_set[64] = {false};
   int dev = 0;
   if (int rc = check_hip(hipGetDevice(&dev), "hipGetDevice")) return rc;
   if (dev < 0 || dev >= 64 || !lds_set[dev]) {
-    if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dl_kernel<T, EPI, AM, NS>),
+    if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dl_kernel<T, EPI, AM>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, L::LDS),
                            "gemm_dl_kernel LDS attribute"))
       return rc;
     if (dev >= 0 && dev < 64) lds_set[dev] = true;
   }
   const dim3 grid((p.N + T::BN - 1) / T::BN, (p.M + T::BM - 1) / T::BM), block(T::THREADS);
-  hipLaunchKernelGGL((gemm_dl_kernel<T, EPI, AM, NS>), grid, block, L::LDS, st, p);
+  hipLaunchKernelGGL((gemm_dl_kernel<T, EPI, AM>), grid, block, L::LDS, st, p);
   YAPD_LAUNCH_CHECK("gemm_dl_kernel launch");
   return YAPD_OK;
 }
@@ -1513,7 +1819,7 @@ using TileM = Tile<128, 128, BK, 4, 2>;  // direct-load mid tile: 8 waves of 32 
 
 template <class T, int EPI, int AM, int BQ>
 int launch_dlq(const GemmParams& p, hipStream_t st) {
-  using L = DlLayout<T, 2>;
+  using L = DlLayout<T>;
   static bool lds_set[64] = {false};
   int dev = 0;
   if (int rc = check_hip(hipGetDevice(&dev), "hipGetDevice")) return rc;
@@ -1530,7 +1836,37 @@ int launch_dlq(const GemmParams& p, hipStream_t st) {
   return YAPD_OK;
 }
 
-using TileW = Tile<64, 64, BK, 1, 1>;     // direct-load one-wave tile (small batches)
+
+template <class T, int EPI, int AM>
+int launch_sk(const GemmParams& p, hipStream_t st) {
+  static bool lds_set[64] = {false};
+  int dev = 0;
+  if (int rc = check_hip(hipGetDevice(&dev), "hipGetDevice")) return rc;
+  if (dev < 0 || dev >= 64 || !lds_set[dev]) {
+    if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_sk_kernel<T, EPI, AM>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS),
+                           "gemm_sk_kernel LDS attribute"))
+      return rc;
+    if (dev >= 0 && dev < 64) lds_set[dev] = true;
+  }
+  const dim3 grid((p.N + T::BN - 1) / T::BN, (p.M + T::BM - 1) / T::BM);
+  hipLaunchKernelGGL((gemm_sk_kernel<T, EPI, AM>), grid, dim3(T::THREADS), T::LDS, st, p);
+  YAPD_LAUNCH_CHECK("gemm_sk_kernel launch");
+  return YAPD_OK;
+}
+
+using Sk16 = SkTile<1, 1, 1, 1, 4, 4, 4, 8>;      //  16 x  16, 1 wave computes, 4 x 16 KB: two per CU
+using Sk32 = SkTile<1, 2, 2, 1, 4, 4, 4, 4>;      //  32 x  32, 2 waves compute, 4 x 32 KB
+using Sk64x32 = SkTile<1, 2, 4, 1, 4, 2, 6, 4>;   //  64 x  32, 4 waves of 16 x 32, 6 x 24 KB
+using Sk64 = SkTile<1, 2, 4, 2, 8, 2, 4, 4>;      //  64 x  64, 8 waves of 16 x 32, 4 x 32 KB
+using Sk128x64 = SkTile<2, 2, 4, 2, 8, 1, 6, 2>;  // 128 x  64, 8 waves of 32 x 32, 6 x 24 KB
+using Sk128 = SkTile<2, 4, 4, 2, 8, 1, 5, 2>;     // 128 x 128, 8 waves of 32 x 64, 5 x 32 KB
+
+template <class T>
+bool sk_fits(const GemmParams& p, int64_t max_tiles) {
+  const int64_t tiles = static_cast<int64_t>((p.M + T::BM - 1) / T::BM) * ((p.N + T::BN - 1) / T::BN);
+  return tiles <= max_tiles && p.K % (64 * T::S) == 0;
+}
 
 // The persistent kernel: one workgroup per CU (fewer when there are fewer tiles).
 template <int EPI, int AM>
@@ -1567,6 +1903,12 @@ int cu_count() {
 
 template <int EPI, int AM, int BQ = 0>
 int launch_gemm(GemmParams p, hipStream_t st) {
+  // The kernels address a tile (up to 256 rows) with 32-bit offsets; wider
+  // pitches take the 128 x 128 kernel with 64-bit addresses.
+  constexpr int64_t kMaxPitch = int64_t{1} << 22;
+  if constexpr (BQ == 0)
+    if (p.ldw > kMaxPitch || (AM == kAPlain && p.lda > kMaxPitch))
+      return launch_dl<TileM, EPI, AM == kAPlain ? kAWide : AM>(p, st);
   // Large tiles once they fill three quarters of the CUs (direct-load kernel;
   // measured at M = 4096: QKV 37.6 -> 33.4 us with 192 tiles, while at 128
   // tiles the 128 x 128 kernel is still faster) or, for the quantised path,
@@ -1586,7 +1928,7 @@ int launch_gemm(GemmParams p, hipStream_t st) {
       const bool narrow_long = (p.N + 255) / 256 <= 8 && p.K >= 2048;
       p.xcd_band = big_tiles <= cu_count() || (EPI == kEpiResidual && narrow_long) ? 1 : 0;
       if constexpr (EPI == kEpiStore) {
-        // the head's last 2 columns (N = 8194) as below: their own one-wave launch
+        // the head's last 2 columns (N = 8194) as below: their own launch
         const int tail = p.N % 256;
         if (tail != 0 && tail <= 64) {
           GemmParams rest = p;
@@ -1594,9 +1936,8 @@ int launch_gemm(GemmParams p, hipStream_t st) {
           rest.W = p.W + static_cast<int64_t>(p.N) * p.ldw;
           rest.C = p.C + p.N;
           rest.N = tail;
-          rest.xcd_band = (p.M + 63) / 64 <= cu_count() ? 1 : 0;
           if (int rc = launch_pt<EPI, AM>(p, st, cu_count())) return rc;
-          return launch_dl<TileW, EPI, AM, 3>(rest, st);
+          return launch_sk<Sk128x64, EPI, AM>(rest, st);
         }
       }
       return launch_pt<EPI, AM>(p, st, cu_count());
@@ -1615,7 +1956,7 @@ int launch_gemm(GemmParams p, hipStream_t st) {
       if constexpr (EPI == kEpiStore) {
         // A last column tile of at most 64 columns that would add a round of
         // 256 x 256 tiles (the speech head: N = 8194 = 32 x 256 + 2, 2112
-        // tiles) goes to a second launch on one-wave 64 x 64 tiles.  Every
+        // tiles) goes to a second launch on 128 x 64 tiles.  Every
         // element keeps the same MFMA and K order, so the output is the same.
         const int64_t row_tiles = (p.M + 255) / 256, cols = p.N / 256, cus = cu_count();
         const int tail = p.N % 256;
@@ -1627,9 +1968,8 @@ int launch_gemm(GemmParams p, hipStream_t st) {
           rest.W = p.W + static_cast<int64_t>(p.N) * p.ldw;
           rest.C = p.C + p.N;
           rest.N = tail;
-          rest.xcd_band = (p.M + 63) / 64 <= cus ? 1 : 0;
           if (int rc = launch_dl<TileD, EPI, AM>(p, st)) return rc;
-          return launch_dl<TileW, EPI, AM, 3>(rest, st);
+          return launch_sk<Sk128x64, EPI, AM>(rest, st);
         }
       }
       return launch_dl<TileD, EPI, AM>(p, st);
@@ -1637,31 +1977,34 @@ int launch_gemm(GemmParams p, hipStream_t st) {
       return launch_dlq<TileD, EPI, AM, BQ>(p, st);
     }
   }
-  // Few tiles (small batches): one-wave 64 x 64 direct-load tiles with two
-  // k-tiles in flight, while they give at most two workgroups per CU
-  // (measured down at M = 256..2048: 46-51 -> 36-41 us; beyond that the
-  // 128 x 128 kernel is faster).
+  // Small and mid M: the smallest tile of gemm_sk_kernel whose grid is at most
+  // one workgroup per CU (two for 16 x 16, of 64 KB of LDS each).  Measured (us,
+  // one graph of 24 calls over 24 weights; one-wave 64 x 64 and three-stage
+  // 128 x 128 tiles before -> now, bit-identical): o M = 64 12.0 -> 3.5, 256
+  // 12.0 -> 4.9, 1000 12.7 -> 7.3, 1900 13.8 -> 9.5, 4096 14.5 -> 13.9; down
+  // M = 64 33.8 -> 6.0, 256 33.4 -> 9.0, 1000 34.5 -> 16.7, 1900 37.8 -> 23.3,
+  // 4096 47.0 -> 38.5; QKV M = 64 12.9 -> 5.1, 512 14.7 -> 10.3; gate/up M = 64
+  // 11.3 -> 6.6, 512 14.5 -> 13.1.  The next larger tile at the same M is slower
+  // by 5 - 50 % (fewer CUs load), the next smaller one by its second round.
+  // Tiles in row bands per XCD where A is the larger operand (down M = 4096
+  // 45.1 -> 38.5 us), else column bands.
+  const int cus = cu_count();
   if constexpr (BQ == 0) {
-    const int64_t wave_tiles = static_cast<int64_t>((p.M + 63) / 64) * ((p.N + 63) / 64);
-    if (wave_tiles <= 2 * cu_count()) {
-      p.xcd_band = wave_tiles <= cu_count() ? 1 : 0;
-      return launch_dl<TileW, EPI, AM, 3>(p, st);
-    }
+    p.xcd_band = p.M > p.N ? 1 : 0;
+    if constexpr (EPI == kEpiStore || EPI == kEpiResidual)
+      if (sk_fits<Sk16>(p, 2 * cus)) return launch_sk<Sk16, EPI, AM>(p, st);
+    if (sk_fits<Sk32>(p, cus)) return launch_sk<Sk32, EPI, AM>(p, st);
+    if (sk_fits<Sk64x32>(p, cus)) return launch_sk<Sk64x32, EPI, AM>(p, st);
+    if (sk_fits<Sk64>(p, cus)) return launch_sk<Sk64, EPI, AM>(p, st);
+    if (sk_fits<Sk128x64>(p, cus)) return launch_sk<Sk128x64, EPI, AM>(p, st);
+    if (sk_fits<Sk128>(p, cus)) return launch_sk<Sk128, EPI, AM>(p, st);
   }
-  // In between, 128 x 128 tiles: the direct-load kernel with 8 waves of 32 x 64
-  // (measured against the register-staged 128 x 128 kernel, same session,
-  // bit-identical: o 18.5 -> 16.9 us and down 53.4 -> 50.4 us at M = 4096,
-  // down 72.9 -> 62.5 us at M = 6144); the quantised path keeps the
-  // register-staged kernel, which dequantises W on its way into LDS.  With at
-  // most one tile per CU a k-tile is too short to cover the load latency, so
-  // three stages keep two tiles in flight (o 16.8 -> 14.3-14.9 us, down
-  // 50.3-51.1 -> 41.0-42.9 us at M = 2304-4096, bit-identical); with more
-  // tiles two stages let two workgroups share a CU, which measured faster
-  // (down 61 vs 83 us at M = 6144).
+  // In between, 128 x 128 tiles of 8 waves, two workgroups of two stages per CU
+  // (down 61 us against 83 us with three stages at M = 6144); the quantised path
+  // keeps the register-staged kernel, which dequantises W on its way into LDS.
   const int64_t small_tiles = static_cast<int64_t>((p.M + 127) / 128) * ((p.N + 127) / 128);
-  p.xcd_band = small_tiles <= cu_count() ? 1 : 0;
+  p.xcd_band = small_tiles <= cus ? 1 : 0;
   if constexpr (BQ == 0) {
-    if (small_tiles <= cu_count()) return launch_dl<TileM, EPI, AM, 3>(p, st);
     return launch_dl<TileM, EPI, AM>(p, st);
   } else {
     // Quantised W: the direct-load kernel on 128 x 128 tiles while the grid
