@@ -11,9 +11,10 @@
 //   * gemm_sk_kernel: 16 x 16 to 128 x 128 tiles, the smallest with at most one
 //     workgroup per CU, as many LDS stages as fit (small and mid M).
 // A and W k-slices go global -> LDS by direct loads.  Affine-quantised W:
-// gemm_dlq_kernel (the direct-load layout with W dequantised from registers
-// into LDS) and, between its two tile sizes, gemm_kernel (register-staged tiles
-// with padded LDS rows).  Every kernel sums K in the same order, so a row's
+// gemm_dlq_kernel (256 x 256 tiles that fill the CUs, W dequantised from registers
+// into LDS), gemm_skq_kernel (up to one workgroup per CU: gemm_sk_kernel's tiles,
+// W dequantised from LDS into LDS) and, between them, gemm_kernel (register-staged
+// 128 x 128 tiles with padded LDS rows).  Every kernel sums K in the same order, so a row's
 // result does not depend on which kernel the batch size selects.  K advances in
 // steps of 64.
 //
@@ -876,20 +877,26 @@ __global__ __launch_bounds__(T::THREADS) void gemm_dl_kernel(const GemmParams p)
 //
 // down, M = 64 (us): one-wave 64 x 64 tiles, three stages 33.8; 16 x 16 tiles
 // with every wait for LDS at lgkmcnt(0) 10.2; counted waits (buffer loads) 6.0.
-template <int TM_, int TN_, int WM_, int WN_, int WAVES_, int S_, int NS_, int P_>
-struct SkTile {
-  static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, WAVES = WAVES_, S = S_, NS = NS_, P = P_;
+template <int TM_, int TN_, int WM_, int WN_, int WAVES_, int S_, int P_>
+struct SkShape {
+  static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, WAVES = WAVES_, S = S_, P = P_;
   static constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
   static constexpr int THREADS = 64 * WAVES;
-  static constexpr int RG = (BM + BN) / 8;  // 1 KB loads per k-tile
-  static constexpr int PW = RG / WAVES;     // of them per wave
-  static constexpr int LPS = PW * S;        // loads per wave and stage
-  static constexpr int KT = RG * 1024;      // bytes of one k-tile
-  static constexpr int STAGE = S * KT;
+  static_assert(WM * WN <= WAVES && (2 * S) % P == 0, "fragment slots must cycle with the stage");
+};
+
+template <int TM_, int TN_, int WM_, int WN_, int WAVES_, int S_, int NS_, int P_>
+struct SkTile : SkShape<TM_, TN_, WM_, WN_, WAVES_, S_, P_> {
+  using Sh = SkShape<TM_, TN_, WM_, WN_, WAVES_, S_, P_>;
+  static constexpr int NS = NS_;
+  static constexpr int RG = (Sh::BM + Sh::BN) / 8;  // 1 KB loads per k-tile
+  static constexpr int PW = RG / Sh::WAVES;         // of them per wave
+  static constexpr int LPS = PW * Sh::S;            // loads per wave and stage
+  static constexpr int KT = RG * 1024;              // bytes of one k-tile
+  static constexpr int STAGE = Sh::S * KT;
   static constexpr int LDS = NS * STAGE;
-  static_assert(PW * WAVES == RG && WM * WN <= WAVES, "loads must split evenly over the waves");
+  static_assert(PW * Sh::WAVES == RG, "loads must split evenly over the waves");
   static_assert((NS - 2) * LPS <= 63 && LDS <= 160 * 1024 && NS >= 3, "vmcnt / LDS limits");
-  static_assert((2 * S) % P == 0, "fragment slots must cycle with the stage");
 };
 
 // Wait until at most N of this wave's loads are in flight, then the workgroup barrier.
@@ -912,169 +919,53 @@ __device__ __forceinline__ void wait_barrier_later(int later) {
   }
 }
 
-template <class T, int EPI, int AM>
-__global__ __launch_bounds__(T::THREADS) void gemm_sk_kernel(const GemmParams p) {
-  extern __shared__ __attribute__((aligned(16))) uint16_t dyn_lds[];
-  char* lds = reinterpret_cast<char*>(dyn_lds);
-  constexpr bool kPair = EPI == kEpiQkv || EPI == kEpiSwiglu;
-  static_assert(!kPair || T::TN % 2 == 0, "pair epilogues need both halves in a wave");
-  const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int wm = wave / T::WN, wn = wave % T::WN;
-  // Workgroup L runs on XCD L % 8: each XCD takes a contiguous run of tiles, in
-  // row bands (columns fastest) with xcd_band, else column bands (rows fastest).
-  int bx, by;
-  {
-    const int C = gridDim.x, R = gridDim.y, n = C * R;
-    const int L = blockIdx.x + C * blockIdx.y;
-    const int x = L % 8;
-    const int t = x * (n / 8) + min(x, n % 8) + L / 8;
-    by = p.xcd_band ? t / C : t % R;
-    bx = p.xcd_band ? t % C : t / R;
-  }
-  const int m0 = by * T::BM;
-  // W row of local column b
-  auto w_col = [&](int b) {
-    if constexpr (kPair) {
-      const int u = bx * (T::BN / 32) + (b >> 5), w = b & 31;
-      return 64 * (u >> 1) + 16 * (u & 1) + (w < 16 ? w : w + 16);
-    } else {
-      return bx * T::BN + b;
-    }
-  };
-  const int kt_n = p.K / 64;
-  const int st_n = kt_n / T::S;
-  // Loads: row groups of 8 rows, T::PW of them per wave.  Through buffer
-  // descriptors from the tile's first row of A and of W on, except for the
-  // shifted A, whose rows come from two arrays.
-  constexpr bool kBuf = AM == kAPlain;
-  const int w0 = kPair ? bx * T::BN & ~63 : bx * T::BN;  // first W row
-  const __amdgpu_buffer_rsrc_t ra = buffer_from(p.A + static_cast<int64_t>(m0) * p.lda);
-  const __amdgpu_buffer_rsrc_t rw = buffer_from(p.W + static_cast<int64_t>(w0) * p.ldw);
-  const uint16_t* src[T::PW];
-  uint32_t ofs[T::PW];
-#pragma unroll
-  for (int j = 0; j < T::PW; ++j) {
-    const int r = (wave * T::PW + j) * 8 + (lane >> 3);
-    const int c = (lane & 7) ^ ((r >> 1) & 7);
-    const bool is_a = (wave * T::PW + j) * 8 < T::BM;
-    if constexpr (kBuf) {
-      const int64_t e = is_a ? static_cast<int64_t>(min(r, p.M - 1 - m0)) * p.lda
-                             : static_cast<int64_t>(min(w_col(r - T::BM), p.N - 1) - w0) * p.ldw;
-      ofs[j] = static_cast<uint32_t>((e + 8 * c) * 2);
-    } else {
-      src[j] = (is_a ? a_row_ptr<AM>(p, min(m0 + r, p.M - 1))
-                     : p.W + static_cast<int64_t>(min(w_col(r - T::BM), p.N - 1)) * p.ldw) + 8 * c;
-    }
-  }
-  auto issue = [&](int st, int slot) {
-    char* dst = lds + slot * T::STAGE + wave * T::PW * 1024;
-#pragma unroll
-    for (int s = 0; s < T::S; ++s) {
-      const int k = (st * T::S + s) * 64;
-#pragma unroll
-      for (int j = 0; j < T::PW; ++j) {
-        if constexpr (kBuf) {
-          load_lds16((wave * T::PW + j) * 8 < T::BM ? ra : rw, ofs[j], 2 * k, dst + s * T::KT + j * 1024);
-        } else {
-          load_lds16(src[j] + k, dst + s * T::KT + j * 1024);
-        }
-      }
-    }
-  };
-  const int tok = lane & 15, sub = 4 * (lane >> 4);
-  // token rows of this lane
-  int pos[T::TM];
-  int prow[T::TM];
-  if constexpr (EPI == kEpiQkv) {
-#pragma unroll
-    for (int i = 0; i < T::TM; ++i) {
-      const int m = min(m0 + (wm * T::TM + i) * 16 + tok, p.M - 1);
-      int r, slot;
-      if (p.tok_row != nullptr) {
-        r = min(max(p.tok_row[m], 0), p.n_rows - 1);
-        slot = m - p.row_start[r];
-      } else {
-        r = m / p.bl;
-        slot = m - r * p.bl;
-      }
-      prow[i] = r;
-      pos[i] = p.pos0[r] + slot;
-    }
-  }
-#pragma unroll
-  for (int s = 0; s + 1 < T::NS; ++s)
-    if (s < st_n) issue(s, s);
+// Workgroup L runs on XCD L % 8: each XCD takes a contiguous run of tiles, in
+// row bands (columns fastest) with xcd_band, else column bands (rows fastest).
+__device__ __forceinline__ int2 sk_tile(const GemmParams& p) {
+  const int C = gridDim.x, R = gridDim.y, n = C * R;
+  const int L = blockIdx.x + C * blockIdx.y;
+  const int x = L % 8;
+  const int t = x * (n / 8) + min(x, n % 8) + L / 8;
+  return p.xcd_band ? make_int2(t % C, t / C) : make_int2(t / R, t % R);
+}
 
-  f32x4_t acc[T::TM][T::TN];
-#pragma unroll
-  for (int i = 0; i < T::TM; ++i)
-#pragma unroll
-    for (int j = 0; j < T::TN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const int sw = (tok >> 1) & 7, cg = lane >> 4;
-  const int a_off = (wm * T::TM * 16 + tok) * 128;
-  const int b_off = (T::BM + wn * T::TN * 16 + tok) * 128;
-  // Fragments are read P k-steps (of 32) ahead of their MFMAs, across stages:
-  // the barrier that hands stage st + 1 over stands P k-steps before the end of
-  // stage st.  Behind it stage st + NS - 1 is requested into the slot of stage
-  // st - 1, whose fragments every wave had consumed when it reached the barrier.
-  constexpr int N = 2 * T::S, P = T::P;
-  bf16x8_t a[P][T::TM], b[P][T::TN];
-  auto read = [&](const char* base, int ks, int q) {
-    const int co = ((4 * (ks & 1) + cg) ^ sw) * 16 + (ks >> 1) * T::KT;
-#pragma unroll
-    for (int j = 0; j < T::TN; ++j) b[q][j] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(base + b_off + j * 2048 + co));
-#pragma unroll
-    for (int i = 0; i < T::TM; ++i) a[q][i] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(base + a_off + i * 2048 + co));
-  };
-  // Hand stage st + 1 over and request stage st + NS - 1 (while there is one).
-  auto hand_over = [&](int st, int slot, auto steady) {
-    if constexpr (decltype(steady)::value) {
-      wait_barrier<(T::NS - 3) * T::LPS>();
-      issue(st + T::NS - 1, slot == 0 ? T::NS - 1 : slot - 1);
-    } else {
-      wait_barrier_later<T::NS - 3, T::LPS>(min(T::NS - 3, st_n - 2 - st));
-    }
-  };
-  wait_barrier_later<T::NS - 2, T::LPS>(min(T::NS - 2, st_n - 1));
-  int slot = 0, st = 0;
-  const auto advance = [&]() { slot = slot + 1 == T::NS ? 0 : slot + 1; };
-  if (wave >= T::WM * T::WN) {  // waves that only load
-    for (; st + T::NS - 1 < st_n; ++st, advance()) hand_over(st, slot, std::true_type{});
-    for (; st + 1 < st_n; ++st) hand_over(st, slot, std::false_type{});
-    return;
+// W row of local column b of column tile bx.
+template <class T, int EPI>
+__device__ __forceinline__ int sk_col(int bx, int b) {
+  if constexpr (EPI == kEpiQkv || EPI == kEpiSwiglu) {
+    const int u = bx * (T::BN / 32) + (b >> 5), w = b & 31;
+    return 64 * (u >> 1) + 16 * (u & 1) + (w < 16 ? w : w + 16);
+  } else {
+    return bx * T::BN + b;
   }
+}
+
+// Position and row of a lane's tokens (qkv).
+template <class T>
+__device__ __forceinline__ void sk_rows(const GemmParams& p, int m0, int wm, int tok, int (&pos)[T::TM],
+                                        int (&prow)[T::TM]) {
 #pragma unroll
-  for (int q = 0; q < P; ++q) read(lds, q, q);
-  // MODE 0: stages follow and loads go out; 1: stages follow; 2: the last stage
-  auto stage = [&](auto mode) {
-    constexpr int MODE = decltype(mode)::value;
-    const char* base = lds + slot * T::STAGE;
-    const char* nbase = lds + (slot + 1 == T::NS ? 0 : slot + 1) * T::STAGE;
-#pragma unroll
-    for (int ks = 0; ks < N; ++ks) {
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < T::TM; ++i)
-#pragma unroll
-        for (int j = 0; j < T::TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[ks % P][j], a[ks % P][i], acc[i][j], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (MODE < 2) {
-        if (ks + P == N) hand_over(st, slot, std::bool_constant<MODE == 0>{});
-      }
-      if (ks + P < N) {
-        read(base, ks + P, ks % P);
-      } else if constexpr (MODE < 2) {
-        read(nbase, ks + P - N, ks % P);
-      }
+  for (int i = 0; i < T::TM; ++i) {
+    const int m = min(m0 + (wm * T::TM + i) * 16 + tok, p.M - 1);
+    int r, slot;
+    if (p.tok_row != nullptr) {
+      r = min(max(p.tok_row[m], 0), p.n_rows - 1);
+      slot = m - p.row_start[r];
+    } else {
+      r = m / p.bl;
+      slot = m - r * p.bl;
     }
-    advance();
-    ++st;
-  };
-  while (st + T::NS - 1 < st_n) stage(std::integral_constant<int, 0>{});
-  while (st + 1 < st_n) stage(std::integral_constant<int, 1>{});
-  stage(std::integral_constant<int, 2>{});
+    prow[i] = r;
+    pos[i] = p.pos0[r] + slot;
+  }
+}
+
+// Epilogues of the 16 x 16 sub-tile kernels, from registers.
+template <class T, int EPI>
+__device__ __forceinline__ void sk_finish(const GemmParams& p, const f32x4_t (&acc)[T::TM][T::TN],
+                                          const int (&pos)[T::TM], const int (&prow)[T::TM], int m0, int bx, int wm,
+                                          int wn, int tok, int sub) {
+  constexpr bool kPair = EPI == kEpiQkv || EPI == kEpiSwiglu;
 #pragma unroll
   for (int i = 0; i < T::TM; ++i) {
     const int m = m0 + (wm * T::TM + i) * 16 + tok;
@@ -1153,10 +1044,426 @@ __global__ __launch_bounds__(T::THREADS) void gemm_sk_kernel(const GemmParams p)
   }
 }
 
+template <class T, int EPI, int AM>
+__global__ __launch_bounds__(T::THREADS) void gemm_sk_kernel(const GemmParams p) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t dyn_lds[];
+  char* lds = reinterpret_cast<char*>(dyn_lds);
+  constexpr bool kPair = EPI == kEpiQkv || EPI == kEpiSwiglu;
+  static_assert(!kPair || T::TN % 2 == 0, "pair epilogues need both halves in a wave");
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wm = wave / T::WN, wn = wave % T::WN;
+  const int2 tile = sk_tile(p);
+  const int bx = tile.x, m0 = tile.y * T::BM;
+  const int kt_n = p.K / 64;
+  const int st_n = kt_n / T::S;
+  // Loads: row groups of 8 rows, T::PW of them per wave.  Through buffer
+  // descriptors from the tile's first row of A and of W on, except for the
+  // shifted A, whose rows come from two arrays.
+  constexpr bool kBuf = AM == kAPlain;
+  const int w0 = kPair ? bx * T::BN & ~63 : bx * T::BN;  // first W row
+  const __amdgpu_buffer_rsrc_t ra = buffer_from(p.A + static_cast<int64_t>(m0) * p.lda);
+  const __amdgpu_buffer_rsrc_t rw = buffer_from(p.W + static_cast<int64_t>(w0) * p.ldw);
+  const uint16_t* src[T::PW];
+  uint32_t ofs[T::PW];
+#pragma unroll
+  for (int j = 0; j < T::PW; ++j) {
+    const int r = (wave * T::PW + j) * 8 + (lane >> 3);
+    const int c = (lane & 7) ^ ((r >> 1) & 7);
+    const bool is_a = (wave * T::PW + j) * 8 < T::BM;
+    if constexpr (kBuf) {
+      const int64_t e = is_a ? static_cast<int64_t>(min(r, p.M - 1 - m0)) * p.lda
+                             : static_cast<int64_t>(min(sk_col<T, EPI>(bx, r - T::BM), p.N - 1) - w0) * p.ldw;
+      ofs[j] = static_cast<uint32_t>((e + 8 * c) * 2);
+    } else {
+      src[j] = (is_a ? a_row_ptr<AM>(p, min(m0 + r, p.M - 1))
+                     : p.W + static_cast<int64_t>(min(sk_col<T, EPI>(bx, r - T::BM), p.N - 1)) * p.ldw) + 8 * c;
+    }
+  }
+  auto issue = [&](int st, int slot) {
+    char* dst = lds + slot * T::STAGE + wave * T::PW * 1024;
+#pragma unroll
+    for (int s = 0; s < T::S; ++s) {
+      const int k = (st * T::S + s) * 64;
+#pragma unroll
+      for (int j = 0; j < T::PW; ++j) {
+        if constexpr (kBuf) {
+          load_lds16((wave * T::PW + j) * 8 < T::BM ? ra : rw, ofs[j], 2 * k, dst + s * T::KT + j * 1024);
+        } else {
+          load_lds16(src[j] + k, dst + s * T::KT + j * 1024);
+        }
+      }
+    }
+  };
+  const int tok = lane & 15, sub = 4 * (lane >> 4);
+  int pos[T::TM], prow[T::TM];
+  if constexpr (EPI == kEpiQkv) sk_rows<T>(p, m0, wm, tok, pos, prow);
+#pragma unroll
+  for (int s = 0; s + 1 < T::NS; ++s)
+    if (s < st_n) issue(s, s);
+
+  f32x4_t acc[T::TM][T::TN];
+#pragma unroll
+  for (int i = 0; i < T::TM; ++i)
+#pragma unroll
+    for (int j = 0; j < T::TN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int sw = (tok >> 1) & 7, cg = lane >> 4;
+  const int a_off = (wm * T::TM * 16 + tok) * 128;
+  const int b_off = (T::BM + wn * T::TN * 16 + tok) * 128;
+  // Fragments are read P k-steps (of 32) ahead of their MFMAs, across stages:
+  // the barrier that hands stage st + 1 over stands P k-steps before the end of
+  // stage st.  Behind it stage st + NS - 1 is requested into the slot of stage
+  // st - 1, whose fragments every wave had consumed when it reached the barrier.
+  constexpr int N = 2 * T::S, P = T::P;
+  bf16x8_t a[P][T::TM], b[P][T::TN];
+  auto read = [&](const char* base, int ks, int q) {
+    const int co = ((4 * (ks & 1) + cg) ^ sw) * 16 + (ks >> 1) * T::KT;
+#pragma unroll
+    for (int j = 0; j < T::TN; ++j) b[q][j] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(base + b_off + j * 2048 + co));
+#pragma unroll
+    for (int i = 0; i < T::TM; ++i) a[q][i] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(base + a_off + i * 2048 + co));
+  };
+  // Hand stage st + 1 over and request stage st + NS - 1 (while there is one).
+  auto hand_over = [&](int st, int slot, auto steady) {
+    if constexpr (decltype(steady)::value) {
+      wait_barrier<(T::NS - 3) * T::LPS>();
+      issue(st + T::NS - 1, slot == 0 ? T::NS - 1 : slot - 1);
+    } else {
+      wait_barrier_later<T::NS - 3, T::LPS>(min(T::NS - 3, st_n - 2 - st));
+    }
+  };
+  wait_barrier_later<T::NS - 2, T::LPS>(min(T::NS - 2, st_n - 1));
+  int slot = 0, st = 0;
+  const auto advance = [&]() { slot = slot + 1 == T::NS ? 0 : slot + 1; };
+  if (wave >= T::WM * T::WN) {  // waves that only load
+    for (; st + T::NS - 1 < st_n; ++st, advance()) hand_over(st, slot, std::true_type{});
+    for (; st + 1 < st_n; ++st) hand_over(st, slot, std::false_type{});
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < P; ++q) read(lds, q, q);
+  // MODE 0: stages follow and loads go out; 1: stages follow; 2: the last stage
+  auto stage = [&](auto mode) {
+    constexpr int MODE = decltype(mode)::value;
+    const char* base = lds + slot * T::STAGE;
+    const char* nbase = lds + (slot + 1 == T::NS ? 0 : slot + 1) * T::STAGE;
+#pragma unroll
+    for (int ks = 0; ks < N; ++ks) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < T::TM; ++i)
+#pragma unroll
+        for (int j = 0; j < T::TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[ks % P][j], a[ks % P][i], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (MODE < 2) {
+        if (ks + P == N) hand_over(st, slot, std::bool_constant<MODE == 0>{});
+      }
+      if (ks + P < N) {
+        read(base, ks + P, ks % P);
+      } else if constexpr (MODE < 2) {
+        read(nbase, ks + P - N, ks % P);
+      }
+    }
+    advance();
+    ++st;
+  };
+  while (st + T::NS - 1 < st_n) stage(std::integral_constant<int, 0>{});
+  while (st + 1 < st_n) stage(std::integral_constant<int, 1>{});
+  stage(std::integral_constant<int, 2>{});
+  sk_finish<T, EPI>(p, acc, pos, prow, m0, bx, wm, wn, tok, sub);
+}
+
+// Affine-quantised W on the same tiles: A as above; W's codes come to LDS by
+// direct loads as they are (a quarter or half of the bf16 bytes), every thread
+// dequantises its share of a stage once per workgroup into a two-slot bf16
+// stage in the fragments' layout (w = scale * q + bias rounded once to bf16, as
+// dq_pair), and the scales and biases of the tile's columns stay in LDS for the
+// whole of K.  Load step i is stage i of A with stage i + 1 of the codes: the
+// barrier that hands A's stage st + 1 over also hands over the codes of
+// st + 2, which are dequantised right behind it into the slot of stage st (all
+// its fragments have been read: the barrier waits for LDS reads too), over the
+// MFMAs up to the next hand-over.  Sums and roundings are gemm_dlq_kernel's.
+template <class T_, int BQ, int NA_>
+struct SkqTile {
+  using T = T_;
+  static constexpr int NA = NA_;                       // stages of A and of codes
+  static constexpr int A_KT = T::BM * 128, B_KT = T::BN * 128, Q_ROW = T::S * 8 * BQ;
+  static constexpr int A_STAGE = T::S * A_KT, B_STAGE = T::S * B_KT, Q_STAGE = T::BN * Q_ROW;
+  static constexpr int LA = A_STAGE / 1024 / T::WAVES;  // 1 KB loads per wave and stage
+  static constexpr int QL = Q_STAGE / 1024;             // 1 KB loads of codes per stage
+  static constexpr int LQ = (QL + T::WAVES - 1) / T::WAVES;
+  static constexpr int U = T::S * T::BN * 8 / T::THREADS;  // runs of 8 codes per thread and stage
+  static constexpr int B0 = NA * A_STAGE, Q0 = B0 + 2 * B_STAGE, S0 = Q0 + NA * Q_STAGE;
+  static_assert(LA * 1024 * T::WAVES == A_STAGE && QL * 1024 == Q_STAGE && QL % LQ == 0, "whole loads per wave");
+  static_assert(U * T::THREADS == T::S * T::BN * 8 && 8 % U == 0, "a thread's codes lie in one row and group");
+  static_assert(NA >= 3 && (NA - 2) * (LA + LQ) + LA <= 63, "vmcnt limit");
+  static int lds(int K) { return S0 + T::BN * (K / 64) * 4; }
+};
+
+// Eight codes (4-bit: one word, 8-bit: two) to bf16.
+template <int BQ>
+__device__ __forceinline__ u32x4_t dq_run(const uint32_t* w, float sc, float bi) {
+  float f[8];
+  if constexpr (BQ == 4) {
+    const uint32_t even = w[0] & 0x0f0f0f0fu, odd = (w[0] >> 4) & 0x0f0f0f0fu;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      f[2 * t] = static_cast<float>((even >> (8 * t)) & 0xffu);
+      f[2 * t + 1] = static_cast<float>((odd >> (8 * t)) & 0xffu);
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < 8; ++t) f[t] = static_cast<float>((w[t >> 2] >> (8 * (t & 3))) & 0xffu);
+  }
+  u32x4_t v;
+#pragma unroll
+  for (int h = 0; h < 4; ++h)
+    v[h] = pack_bf16x2(__builtin_fmaf(sc, f[2 * h], bi), __builtin_fmaf(sc, f[2 * h + 1], bi));
+  return v;
+}
+
+template <class Q, int EPI, int BQ>
+__global__ __launch_bounds__(Q::T::THREADS) void gemm_skq_kernel(const GemmParams p) {
+  using T = typename Q::T;
+  extern __shared__ __attribute__((aligned(16))) uint16_t dyn_lds[];
+  char* lds = reinterpret_cast<char*>(dyn_lds);
+  constexpr bool kPair = EPI == kEpiQkv || EPI == kEpiSwiglu;
+  static_assert(!kPair || T::TN % 2 == 0, "pair epilogues need both halves in a wave");
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wm = wave / T::WN, wn = wave % T::WN;
+  const int2 tile = sk_tile(p);
+  const int bx = tile.x, m0 = tile.y * T::BM;
+  const int kt_n = p.K / 64;
+  const int st_n = kt_n / T::S;
+  const int w0 = kPair ? bx * T::BN & ~63 : bx * T::BN;  // first W row
+
+  // scales and biases: (kt, row) as one word at kt * BN + (row ^ (kt & 15)); a
+  // batch's loads are in flight over the first direct loads
+  uint32_t* sb = reinterpret_cast<uint32_t*>(lds + Q::S0);
+  uint32_t sv[4];
+  auto sb_load = [&](int e0) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int e = e0 + t * T::THREADS + tid;
+      const int row = e / kt_n, kt = e - row * kt_n;
+      const int64_t at = static_cast<int64_t>(min(sk_col<T, EPI>(bx, min(row, T::BN - 1)), p.N - 1)) * kt_n + kt;
+      sv[t] = p.qscale[at] | static_cast<uint32_t>(p.qbias[at]) << 16;
+    }
+  };
+  auto sb_store = [&](int e0) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int e = e0 + t * T::THREADS + tid;
+      const int row = e / kt_n, kt = e - row * kt_n;
+      if (row < T::BN) sb[kt * T::BN + (row ^ (kt & 15))] = sv[t];
+    }
+  };
+  sb_load(0);
+
+  const __amdgpu_buffer_rsrc_t ra = buffer_from(p.A + static_cast<int64_t>(m0) * p.lda);
+  const __amdgpu_buffer_rsrc_t rq =
+      buffer_from(reinterpret_cast<const uint16_t*>(p.Wq + static_cast<int64_t>(w0) * p.ldq));
+  uint32_t a_ofs[Q::LA], q_ofs[Q::LQ];
+#pragma unroll
+  for (int j = 0; j < Q::LA; ++j) {
+    const int g = wave * Q::LA + j;  // 1 KB group of the stage: k-tile g / (BM / 8), rows 8 (g % (BM / 8)) ..
+    const int r = g % (T::BM / 8) * 8 + (lane >> 3);
+    const int c = (lane & 7) ^ ((r >> 1) & 7);
+    a_ofs[j] = static_cast<uint32_t>((static_cast<int64_t>(min(r, p.M - 1 - m0)) * p.lda + 64 * (g / (T::BM / 8)) + 8 * c) * 2);
+  }
+  const bool loads_q = wave * Q::LQ < Q::QL;
+#pragma unroll
+  for (int j = 0; j < Q::LQ; ++j) {
+    const int b = (wave * Q::LQ + j) * 1024 + lane * 16;  // byte of the code stage: row b / Q_ROW
+    const int row = min(b / Q::Q_ROW, T::BN - 1);
+    q_ofs[j] = static_cast<uint32_t>((min(sk_col<T, EPI>(bx, row), p.N - 1) - w0) * p.ldq * 4 + b % Q::Q_ROW);
+  }
+  auto issue_a = [&](int st, int slot) {
+#pragma unroll
+    for (int j = 0; j < Q::LA; ++j)
+      load_lds16(ra, a_ofs[j], st * (T::S * 128), lds + slot * Q::A_STAGE + (wave * Q::LA + j) * 1024);
+  };
+  auto issue_q = [&](int st, int slot) {
+    if (!loads_q) return;
+#pragma unroll
+    for (int j = 0; j < Q::LQ; ++j)
+      load_lds16(rq, q_ofs[j], min(st, st_n - 1) * Q::Q_ROW,
+                 lds + Q::Q0 + slot * Q::Q_STAGE + (wave * Q::LQ + j) * 1024);
+  };
+  // at most n load steps (and EXTRA loads) of this wave in flight, its LDS accesses done; then the barrier
+  auto wait_steps = [&](auto n) {
+    constexpr int kN = decltype(n)::value;
+    if (loads_q) {
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kN * (Q::LA + Q::LQ)) : "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kN * Q::LA) : "memory");
+    }
+  };
+
+  // Dequantisation of one stage: this thread's U runs of 8 codes of one row and
+  // k-tile, two steps (codes to registers; bf16 to the stage slot).
+  constexpr int TPR = 8 / Q::U;  // threads per row and k-tile
+  const int d_part = tid % TPR, d_row = tid / TPR % T::BN, d_kt = tid / (TPR * T::BN);
+  constexpr int WPT = Q::U * BQ / 4;  // words of codes
+  uint32_t dq_w[WPT], dq_s;
+  auto dq_read = [&](int st, int slot) {
+    const char* src = lds + Q::Q0 + slot * Q::Q_STAGE + d_row * Q::Q_ROW + d_kt * (8 * BQ) + d_part * (Q::U * BQ);
+    if constexpr (WPT == 1) {
+      dq_w[0] = *reinterpret_cast<const uint32_t*>(src);
+    } else if constexpr (WPT == 2) {
+      const u32x2_t v = *reinterpret_cast<const u32x2_t*>(src);
+      dq_w[0] = v[0], dq_w[1] = v[1];
+    } else {
+#pragma unroll
+      for (int t = 0; t < WPT; t += 4) {
+        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(src + 4 * t);
+        dq_w[t] = v[0], dq_w[t + 1] = v[1], dq_w[t + 2] = v[2], dq_w[t + 3] = v[3];
+      }
+    }
+    const int kt = st * T::S + d_kt;
+    dq_s = sb[kt * T::BN + (d_row ^ (kt & 15))];
+  };
+  auto dq_write = [&](int st) {
+    const float sc = f16_to_f32(static_cast<uint16_t>(dq_s)), bi = f16_to_f32(static_cast<uint16_t>(dq_s >> 16));
+    char* dst = lds + Q::B0 + (st & 1) * Q::B_STAGE + d_kt * Q::B_KT + d_row * 128;
+#pragma unroll
+    for (int u = 0; u < Q::U; ++u)
+      *reinterpret_cast<u32x4_t*>(dst + ((d_part * Q::U + u) ^ ((d_row >> 1) & 7)) * 16) =
+          dq_run<BQ>(dq_w + u * (BQ / 4), sc, bi);
+  };
+
+  const int tok = lane & 15, sub = 4 * (lane >> 4);
+  int pos[T::TM], prow[T::TM];
+  if constexpr (EPI == kEpiQkv) sk_rows<T>(p, m0, wm, tok, pos, prow);
+
+  // Prologue: codes 0, then steps 0 .. NA - 2 (A i, codes i + 1), A of step NA - 1 and, once the
+  // slot of codes 0 is free, its codes.
+  constexpr int NA = Q::NA;
+  issue_q(0, 0);
+#pragma unroll
+  for (int i = 0; i + 1 < NA; ++i) {
+    issue_a(i, i);
+    issue_q(i + 1, i + 1);
+  }
+  issue_a(NA - 1, NA - 1);
+  sb_store(0);
+  for (int e0 = 4 * T::THREADS; e0 < T::BN * kt_n; e0 += 4 * T::THREADS) {
+    sb_load(e0);
+    sb_store(e0);
+  }
+  if (loads_q) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NA - 2) * (Q::LA + Q::LQ) + Q::LA) : "memory");
+  } else {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NA - 1) * Q::LA) : "memory");
+  }
+  dq_read(0, 0);
+  dq_write(0);
+  dq_read(1, 1);
+  dq_write(1);
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  issue_q(NA, 0);
+
+  f32x4_t acc[T::TM][T::TN];
+#pragma unroll
+  for (int i = 0; i < T::TM; ++i)
+#pragma unroll
+    for (int j = 0; j < T::TN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int sw = (tok >> 1) & 7, cg = lane >> 4;
+  const int a_off = (wm * T::TM * 16 + tok) * 128;
+  const int b_off = Q::B0 + (wn * T::TN * 16 + tok) * 128;
+  constexpr int N = 2 * T::S, P = T::P;
+  bf16x8_t a[P][T::TM], b[P][T::TN];
+  auto read = [&](int st, int slot, int ks, int q) {
+    const int co = ((4 * (ks & 1) + cg) ^ sw) * 16;
+    const char* bb = lds + (st & 1) * Q::B_STAGE + (ks >> 1) * Q::B_KT + b_off + co;
+    const char* ab = lds + slot * Q::A_STAGE + (ks >> 1) * Q::A_KT + a_off + co;
+#pragma unroll
+    for (int j = 0; j < T::TN; ++j) b[q][j] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(bb + j * 2048));
+#pragma unroll
+    for (int i = 0; i < T::TM; ++i) a[q][i] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(ab + i * 2048));
+  };
+  // slot: st % NA.  Hand A's stage st + 1 and the codes of st + 2 over; request
+  // step st + NA into the slots of A's stage st and of the codes of st + 1.
+  auto wait_later = [&](int later) {
+    if constexpr (NA >= 5) {
+      if (later >= 3) {
+        wait_steps(std::integral_constant<int, NA >= 5 ? 3 : 0>{});
+        return;
+      }
+    }
+    if constexpr (NA >= 4) {
+      if (later == 2) {
+        wait_steps(std::integral_constant<int, NA >= 4 ? 2 : 0>{});
+        return;
+      }
+    }
+    if (later >= 1) {
+      wait_steps(std::integral_constant<int, 1>{});
+    } else {
+      wait_steps(std::integral_constant<int, 0>{});
+    }
+  };
+  static_assert(NA <= 5, "waits are written out for at most five stages");
+  const auto next = [](int s) { return s + 1 == NA ? 0 : s + 1; };
+  auto hand_over = [&](int st, int slot, auto steady) {
+    if constexpr (decltype(steady)::value) {
+      wait_steps(std::integral_constant<int, NA - 2>{});
+      issue_a(st + NA, slot);
+      issue_q(st + NA + 1, next(slot));
+    } else {
+      wait_later(min(NA - 2, st_n - 2 - st));
+    }
+    if (st + 2 < st_n) dq_read(st + 2, next(next(slot)));
+  };
+  int slot = 0, st = 0;
+  if (wave >= T::WM * T::WN) {  // waves that only load and dequantise
+    for (; st + NA < st_n; ++st, slot = next(slot)) {
+      hand_over(st, slot, std::true_type{});
+      if (st + 2 < st_n) dq_write(st + 2);
+    }
+    for (; st + 1 < st_n; ++st, slot = next(slot)) {
+      hand_over(st, slot, std::false_type{});
+      if (st + 2 < st_n) dq_write(st + 2);
+    }
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < P; ++q) read(0, 0, q, q);
+  // MODE 0: stages follow and loads go out; 1: stages follow; 2: the last stage
+  auto stage = [&](auto mode) {
+    constexpr int MODE = decltype(mode)::value;
+#pragma unroll
+    for (int ks = 0; ks < N; ++ks) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < T::TM; ++i)
+#pragma unroll
+        for (int j = 0; j < T::TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[ks % P][j], a[ks % P][i], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (MODE < 2) {
+        if (ks + P == N) hand_over(st, slot, std::bool_constant<MODE == 0>{});
+        if (ks + P == N + 1 && st + 2 < st_n) dq_write(st + 2);
+      }
+      if (ks + P < N) {
+        read(st, slot, ks + P, ks % P);
+      } else if constexpr (MODE < 2) {
+        read(st + 1, next(slot), ks + P - N, ks % P);
+      }
+    }
+    slot = next(slot);
+    ++st;
+  };
+  while (st + NA < st_n) stage(std::integral_constant<int, 0>{});
+  while (st + 1 < st_n) stage(std::integral_constant<int, 1>{});
+  stage(std::integral_constant<int, 2>{});
+  sk_finish<T, EPI>(p, acc, pos, prow, m0, bx, wm, wn, tok, sub);
+}
+
 // Affine-quantised W on the direct-load layout: A moves global -> LDS by
-// direct loads as in gemm_dl_kernel; W's codes (one 16-byte chunk per code
-// row and k-half or quarter -- 8-byte chunks where 16-byte ones would not
-// give every thread one: 4-bit codes on 128-column tiles), scales and biases
+// direct loads as in gemm_dl_kernel; W's codes (16-byte chunks), scales and biases
 // come into registers one k-tile ahead, and after the k-tile's MFMAs each thread dequantises its
 // chunk (w = scale * q + bias, rounded once to bf16, as in gemm_kernel) and
 // writes it into the next stage's B tile in the same swizzled layout, so the
@@ -1189,11 +1496,10 @@ __global__ __launch_bounds__(T::THREADS) void gemm_dlq_kernel(const GemmParams p
     for (int j = 0; j < L::LA; ++j) load_lds16(a_src[j] + kt * T::BK, a_dst + j * 1024);
   };
 
-  // W codes: a chunk of QB bytes holds QVALS codes of one row; a row's k-tile
-  // (one quantisation group of 64) is QCH chunks; each thread owns CQ chunks.
-  constexpr int QB = (T::BN * (T::BK * BQ / 128)) % T::THREADS == 0 ? 16 : 8;
-  constexpr int QW = QB / 4;  // 32-bit words per chunk
-  constexpr int QVALS = QB * 8 / BQ;
+  // W codes: a 16-byte chunk holds QVALS codes of one row; a row's k-tile (one
+  // quantisation group of 64) is QCH chunks; each thread owns CQ chunks.
+  constexpr int QW = 4;  // 32-bit words per chunk
+  constexpr int QVALS = 128 / BQ;
   constexpr int QCH = T::BK / QVALS;
   constexpr int CQ = T::BN * QCH / T::THREADS;
   static_assert(CQ >= 1 && CQ * T::THREADS == T::BN * QCH, "quantised tile loads must divide evenly");
@@ -1218,15 +1524,9 @@ __global__ __launch_bounds__(T::THREADS) void gemm_dlq_kernel(const GemmParams p
 #pragma unroll
     for (int c = 0; c < CQ; ++c) {
       const uint32_t* src = q_src[c] + kt * T::BK * BQ / 32;
-      if constexpr (QW == 4) {
-        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(src);
+      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(src);
 #pragma unroll
-        for (int w = 0; w < 4; ++w) rq[c][w] = v[w];
-      } else {
-        const uint2 v = *reinterpret_cast<const uint2*>(src);
-        rq[c][0] = v.x;
-        rq[c][1] = v.y;
-      }
+      for (int w = 0; w < QW; ++w) rq[c][w] = v[w];
       rs[c] = s_src[c][kt];
       rz[c] = z_src[c][kt];
     }
@@ -1783,6 +2083,10 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const NormParams p) {
 
 bool al16(const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15u) == 0; }
 
+constexpr int kLdsBytes = 160 * 1024;  // per CU
+// Row pitch (elements) up to which a tile of 256 rows is addressed with 32-bit offsets.
+constexpr int64_t kMaxPitch = int64_t{1} << 22;
+
 using TileS = Tile<128, 128, BK, 2, 2>;  // small M: more workgroups
 
 template <class T, int EPI, int AM, int BQ>
@@ -1868,6 +2172,40 @@ bool sk_fits(const GemmParams& p, int64_t max_tiles) {
   return tiles <= max_tiles && p.K % (64 * T::S) == 0;
 }
 
+template <class Q, int EPI, int BQ>
+int launch_skq(const GemmParams& p, hipStream_t st) {
+  using T = typename Q::T;
+  static bool lds_set[64] = {false};
+  int dev = 0;
+  if (int rc = check_hip(hipGetDevice(&dev), "hipGetDevice")) return rc;
+  if (dev < 0 || dev >= 64 || !lds_set[dev]) {
+    if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_skq_kernel<Q, EPI, BQ>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes),
+                           "gemm_skq_kernel LDS attribute"))
+      return rc;
+    if (dev >= 0 && dev < 64) lds_set[dev] = true;
+  }
+  const dim3 grid((p.N + T::BN - 1) / T::BN, (p.M + T::BM - 1) / T::BM);
+  hipLaunchKernelGGL((gemm_skq_kernel<Q, EPI, BQ>), grid, dim3(T::THREADS), Q::lds(p.K), st, p);
+  YAPD_LAUNCH_CHECK("gemm_skq_kernel launch");
+  return YAPD_OK;
+}
+
+template <int BQ> using Skq16 = SkqTile<SkShape<1, 1, 1, 1, 8, 4, 8>, BQ, 4>;       //  16 x  16
+template <int BQ> using Skq32x16 = SkqTile<SkShape<1, 1, 2, 1, 8, 4, 8>, BQ, 4>;    //  32 x  16, 2 waves compute
+template <int BQ> using Skq32 = SkqTile<SkShape<1, 2, 2, 1, 8, 4, 4>, BQ, 4>;       //  32 x  32, 2 waves of 16 x 32
+template <int BQ> using Skq64x32 = SkqTile<SkShape<1, 2, 4, 1, 8, 2, 4>, BQ, 5>;    //  64 x  32, 4 waves of 16 x 32
+template <int BQ> using Skq64 = SkqTile<SkShape<2, 2, 2, 2, 16, 2, 4>, BQ, 4>;      //  64 x  64, 4 waves of 32 x 32
+template <int BQ> using Skq128x64 = SkqTile<SkShape<4, 2, 2, 2, 16, 2, 2>, BQ, 3>;  // 128 x  64, 4 waves of 64 x 32
+template <int BQ> using Skq128 = SkqTile<SkShape<4, 2, 2, 4, 16, 1, 2>, BQ, 3>;     // 128 x 128, 8 waves of 64 x 32
+
+// The tile gives at most max_tiles workgroups, and K suits its stages and fits the scales' LDS.
+template <class Q>
+bool skq_fits(const GemmParams& p, int64_t max_tiles) {
+  return sk_fits<typename Q::T>(p, max_tiles) && p.K / (64 * Q::T::S) >= Q::NA && p.K <= (1 << 16) &&
+         Q::lds(p.K) <= kLdsBytes && p.lda <= kMaxPitch;
+}
+
 // The persistent kernel: one workgroup per CU (fewer when there are fewer tiles).
 template <int EPI, int AM>
 int launch_pt(const GemmParams& p, hipStream_t st, int cus) {
@@ -1903,9 +2241,7 @@ int cu_count() {
 
 template <int EPI, int AM, int BQ = 0>
 int launch_gemm(GemmParams p, hipStream_t st) {
-  // The kernels address a tile (up to 256 rows) with 32-bit offsets; wider
-  // pitches take the 128 x 128 kernel with 64-bit addresses.
-  constexpr int64_t kMaxPitch = int64_t{1} << 22;
+  // wider pitches take the 128 x 128 kernel with 64-bit addresses
   if constexpr (BQ == 0)
     if (p.ldw > kMaxPitch || (AM == kAPlain && p.lda > kMaxPitch))
       return launch_dl<TileM, EPI, AM == kAPlain ? kAWide : AM>(p, st);
@@ -2007,11 +2343,28 @@ int launch_gemm(GemmParams p, hipStream_t st) {
   if constexpr (BQ == 0) {
     return launch_dl<TileM, EPI, AM>(p, st);
   } else {
-    // Quantised W: the direct-load kernel on 128 x 128 tiles while the grid
-    // has at most one tile per CU (M = 256-4096, bit-identical: down 4-bit
-    // 58.1 -> 44.7 us at M = 256, 78.0 -> 72.5 us at M = 4096); larger grids
-    // keep the register-staged kernel (o at M = 8192: 29.3 vs 32.5 us).
-    if (small_tiles <= cu_count()) return launch_dlq<TileM, EPI, AM, BQ>(p, st);
+    // Quantised W: the same rule on gemm_skq_kernel's tiles.  Measured (us, one
+    // graph of 24 calls over 12 weights, 4 bits; 128 x 128 tiles of
+    // gemm_dlq_kernel before -> now, bit-identical): QKV M = 64 12.9 -> 5.9, 400
+    // 14.1 -> 10.8; o M = 64 12.7 -> 4.3, 900 14.8 -> 8.1; gate/up M = 64 14.1 ->
+    // 6.9; down M = 64 47.3 -> 8.1, 400 48.9 -> 16.0, 900 52.6 -> 21.1, 1900 69.7
+    // -> 27.3, 4095 69.7 -> 45.9 (8 bits within 3 %).  16 waves in the larger
+    // tiles: every wave dequantises, and few compute waves of 64 x 32 read the
+    // fewest fragments from LDS (128 x 64 tiles, down M = 1900: 8 waves of 32 x 32
+    // 32.4, 4 of 64 x 32 27.3).
+    p.xcd_band = p.M > p.N ? 1 : 0;
+    if constexpr (EPI == kEpiStore || EPI == kEpiResidual) {
+      if (skq_fits<Skq16<BQ>>(p, cus)) return launch_skq<Skq16<BQ>, EPI, BQ>(p, st);
+      if (skq_fits<Skq32x16<BQ>>(p, cus)) return launch_skq<Skq32x16<BQ>, EPI, BQ>(p, st);
+    }
+    if (skq_fits<Skq32<BQ>>(p, cus)) return launch_skq<Skq32<BQ>, EPI, BQ>(p, st);
+    if (skq_fits<Skq64x32<BQ>>(p, cus)) return launch_skq<Skq64x32<BQ>, EPI, BQ>(p, st);
+    if (skq_fits<Skq64<BQ>>(p, cus)) return launch_skq<Skq64<BQ>, EPI, BQ>(p, st);
+    if (skq_fits<Skq128x64<BQ>>(p, cus)) return launch_skq<Skq128x64<BQ>, EPI, BQ>(p, st);
+    if (skq_fits<Skq128<BQ>>(p, cus)) return launch_skq<Skq128<BQ>, EPI, BQ>(p, st);
+    // Larger grids (o at M = 8192: 29.3 us against 32.5 with gemm_dlq_kernel's
+    // 128 x 128 tiles) and K of fewer k-tiles than the rings hold.
+    p.xcd_band = small_tiles <= cus ? 1 : 0;
     return launch_tile<TileS, EPI, AM, BQ>(p, st);
   }
 }
