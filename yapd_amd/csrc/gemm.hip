@@ -2159,12 +2159,14 @@ int launch_sk(const GemmParams& p, hipStream_t st) {
   return YAPD_OK;
 }
 
-using Sk16 = SkTile<1, 1, 1, 1, 4, 4, 4, 8>;      //  16 x  16, 1 wave computes, 4 x 16 KB: two per CU
-using Sk32 = SkTile<1, 2, 2, 1, 4, 4, 4, 4>;      //  32 x  32, 2 waves compute, 4 x 32 KB
+using Sk16 = SkTile<1, 1, 1, 1, 4, 4, 4, 8>;      //  16 x  16, 1 wave computes, 4 x 16 KB
+using Sk32x16 = SkTile<1, 1, 2, 1, 6, 4, 4, 8>;   //  32 x  16, 2 waves compute, 4 x 24 KB
+using Sk32 = SkTile<1, 1, 2, 2, 4, 4, 4, 8>;      //  32 x  32, 4 waves of 16 x 16, 4 x 32 KB
+using Sk32p = SkTile<1, 2, 2, 1, 4, 4, 4, 4>;     //  the same for pair epilogues, 2 waves of 16 x 32 compute
 using Sk64x32 = SkTile<1, 2, 4, 1, 4, 2, 6, 4>;   //  64 x  32, 4 waves of 16 x 32, 6 x 24 KB
 using Sk64 = SkTile<1, 2, 4, 2, 8, 2, 4, 4>;      //  64 x  64, 8 waves of 16 x 32, 4 x 32 KB
-using Sk128x64 = SkTile<2, 2, 4, 2, 8, 1, 6, 2>;  // 128 x  64, 8 waves of 32 x 32, 6 x 24 KB
-using Sk128 = SkTile<2, 4, 4, 2, 8, 1, 5, 2>;     // 128 x 128, 8 waves of 32 x 64, 5 x 32 KB
+using Sk128x64 = SkTile<4, 2, 2, 2, 8, 1, 6, 2>;  // 128 x  64, 4 waves of 64 x 32 compute, 6 x 24 KB
+using Sk128 = SkTile<4, 4, 2, 2, 8, 1, 5, 2>;     // 128 x 128, 4 waves of 64 x 64 compute, 5 x 32 KB
 
 template <class T>
 bool sk_fits(const GemmParams& p, int64_t max_tiles) {
@@ -2327,9 +2329,13 @@ int launch_gemm(GemmParams p, hipStream_t st) {
   const int cus = cu_count();
   if constexpr (BQ == 0) {
     p.xcd_band = p.M > p.N ? 1 : 0;
-    if constexpr (EPI == kEpiStore || EPI == kEpiResidual)
-      if (sk_fits<Sk16>(p, 2 * cus)) return launch_sk<Sk16, EPI, AM>(p, st);
-    if (sk_fits<Sk32>(p, cus)) return launch_sk<Sk32, EPI, AM>(p, st);
+    if constexpr (EPI == kEpiStore || EPI == kEpiResidual) {
+      if (sk_fits<Sk16>(p, cus)) return launch_sk<Sk16, EPI, AM>(p, st);
+      if (sk_fits<Sk32x16>(p, cus)) return launch_sk<Sk32x16, EPI, AM>(p, st);
+      if (sk_fits<Sk32>(p, cus)) return launch_sk<Sk32, EPI, AM>(p, st);
+    } else {
+      if (sk_fits<Sk32p>(p, cus)) return launch_sk<Sk32p, EPI, AM>(p, st);
+    }
     if (sk_fits<Sk64x32>(p, cus)) return launch_sk<Sk64x32, EPI, AM>(p, st);
     if (sk_fits<Sk64>(p, cus)) return launch_sk<Sk64, EPI, AM>(p, st);
     if (sk_fits<Sk128x64>(p, cus)) return launch_sk<Sk128x64, EPI, AM>(p, st);
