@@ -1,0 +1,78 @@
+"""Few rows (attn_ring_kernel): both sides of its limit, rows with fewer chunks than the ring and
+more pages than one page-table load, every tile count, causal blocks and split items, against fp64 attention
+on the same bf16 inputs; and bit for bit the rows of a call large enough for attn_paged_kernel.
+
+Bound: bf16 has 8 significant bits, so a rounding moves a value by at most 2^-8 of it.  P is rounded before
+P V and the result once more: 2^-8 * sum(p |v|) + 2^-8 * |out| <= 2.1 * 2^-8 * sum(p |v|) with room for the
+fp32 sums (the one-wave kernel reaches 1.65 * 2^-8 on the same inputs)."""
+
+import pytest
+import torch
+
+from yapd_amd.paged import AttnPlan
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+
+def run(dev, rows, bl, H, lens, causal=False, **plan_kw):
+    g = torch.Generator(device=dev).manual_seed(rows * 100 + bl + H)
+    cols = (max(lens) + 15) // 16 + 1
+    table = torch.randperm(rows * cols, generator=g, device=dev).to(torch.int32).view(rows, cols)
+    pool = torch.randn(rows * cols, 2, H, 1024, generator=g, device=dev).to(BF)
+    q = torch.randn(rows, bl, H, 64, generator=g, device=dev).to(BF) * 2
+    out = torch.full_like(q, float("nan"))
+    plan = AttnPlan(lens, bl, H, torch.device(dev), **plan_kw)
+    plan.run(q, pool, table, out, 0.125, causal=causal)
+    for r, n in enumerate(lens):
+        pages = table[r, : (n + 15) // 16].long()
+        k = pool[pages, 0].view(-1, H, 16, 64).transpose(0, 1).reshape(H, -1, 64)[:, :n].double()
+        v = pool[pages, 1].view(-1, H, 64, 16).permute(1, 0, 3, 2).reshape(H, -1, 64)[:, :n].double()
+        s = torch.matmul(q[r].double().transpose(0, 1), k.transpose(1, 2).contiguous()) * 0.125
+        if causal:
+            i = torch.arange(bl, device=dev)[:, None] + n - bl
+            s = s.masked_fill(torch.arange(n, device=dev)[None] > i, float("-inf"))
+        p = s.softmax(-1)
+        ref, mag = torch.matmul(p, v).transpose(0, 1), torch.matmul(p, v.abs()).transpose(0, 1)
+        assert ((out[r].double() - ref).abs() <= 2.1 * 2.0 ** -8 * mag + 1e-6).all(), (r, n)
+    return plan
+
+
+@pytest.mark.parametrize("bl", [1, 16, 17, 32, 48, 64])
+@pytest.mark.parametrize("rows", [1, 3, 17, 96])  # H = 16: 96 rows are the limit
+@pytest.mark.parametrize("causal", [False, True])
+def test_few_rows(dev, rows, bl, causal):
+    lens = [max(bl, n) for n in ([1, 31, 32, 33, 64, 97, 129, 300, 541] * 11)[:rows]]
+    run(dev, rows, bl, 16, lens, causal)
+
+
+@pytest.mark.parametrize("H", [4, 8, 32])
+def test_head_counts(dev, H):
+    run(dev, 5, 32, H, [40, 700, 33, 64, 250])
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_split_rows(dev, causal):
+    """Rows split over work items, and items past 64 pages."""
+    plan = run(dev, 3, 16, 16, [2000, 50, 700], causal, target_items=64, min_split_keys=64)
+    assert plan.n_slots > 0
+    run(dev, 2, 16, 16, [3001, 1050], causal, min_split_keys=4096)
+
+
+@pytest.mark.parametrize("bl", [8, 32, 48, 64])
+@pytest.mark.parametrize("causal", [False, True])
+def test_rows_equal_those_of_a_large_call(dev, bl, causal):
+    """97 rows run on attn_paged_kernel, their first 5 alone on the ring."""
+    H, lens = 16, [max(bl, n) for n in ([70, 33, 1100, 64, 419] * 20)[:97]]
+    g = torch.Generator(device=dev).manual_seed(bl)
+    cols = (max(lens) + 15) // 16
+    table = torch.randperm(97 * cols, generator=g, device=dev).to(torch.int32).view(97, cols)
+    pool = torch.randn(97 * cols, 2, H, 1024, generator=g, device=dev).to(BF)
+    q = torch.randn(97, bl, H, 64, generator=g, device=dev).to(BF)
+    outs = []
+    for n in (97, 5):
+        out = torch.full_like(q[:n], float("nan"))
+        plan = AttnPlan(lens[:n], bl, H, torch.device(dev), min_split_keys=2048)
+        plan.run(q[:n], pool, table[:n], out, 0.125, causal=causal)
+        outs.append(out)
+    assert torch.equal(outs[0][:5], outs[1])

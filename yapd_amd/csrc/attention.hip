@@ -6,7 +6,7 @@
 // engines/torch_sdpa.py:299-307 uses a zero mask).  The block's own K/V are
 // already in the pool (written by the QKV epilogue or yapd_kv_write).
 //
-// Work decomposition: a workgroup of four waves serves one (row, key range)
+// Work decomposition (attn_paged_kernel; few rows: attn_ring_kernel): a workgroup of four waves serves one (row, key range)
 // work item for four heads, one head per wave, so a workgroup streams
 // 4 heads x (2 KiB K + 2 KiB V) contiguous bytes per page.  The H / 4
 // workgroups of one item are consecutive in the 1-D grid: they are dispatched
@@ -32,6 +32,7 @@
 #include "attention.h"
 #include "common.h"
 #include "kv_layout.h"
+#include "lds_dma.h"
 
 namespace yapd {
 namespace {
@@ -103,14 +104,142 @@ __device__ __forceinline__ float sum_xor16_32(float v) {
   return b.x + b.y;
 }
 
-// Occupancy by query tiles, measured (no spills at any of them): three and
-// four tiles (blocks of 33-64 queries, the 64-token prefill chunks) are held
-// to two waves per SIMD -- without the bound the compiler takes 222 VGPRs +
-// 64 AGPRs for four tiles, one wave per SIMD (prefill 294 -> 280 ms).  One and
-// two tiles keep the compiler's three and two: one more wave per SIMD made
-// two tiles 3.7 % slower, and one tile 2 % faster on 256 rows of <= 540 keys
-// but 4.5 % slower on the 30-layer stress shape (prefixes up to 2048 keys):
-// more resident waves are more scattered page streams at once.
+// One 32-key chunk of a 16-query tile: S^T = K Q^T, the online-softmax step, O^T += V^T P^T.  A lane
+// serves query n = lane & 15 with keys k0 + 8g .. + 7; with mask, keys from klim on are left out.
+__device__ __forceinline__ void attn_chunk(const bf16x8_t (&qf)[2], const u32x4_t (&kf)[2][2], const u32x4_t (&vf)[4],
+                                           float scale_log2, bool mask, int key0, int klim, float& m, float& l,
+                                           f32x4_t (&o)[4]) {
+  f32x4_t s[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+    s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kf[t][0]), qf[0], f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+    s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kf[t][1]), qf[1], s[t], 0, 0, 0);
+  // s[t][j] = S[q = n][key 8g + 4t + j]
+  float sv[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) sv[i] = s[i >> 2][i & 3] * scale_log2;
+  if (mask) {  // uniform
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sv[i] = key0 + i >= klim ? -INFINITY : sv[i];
+  }
+  float cm = sv[0];
+#pragma unroll
+  for (int i = 1; i < 8; ++i) cm = fmaxf(cm, sv[i]);
+  cm = max_xor16_32(cm);
+  const float mn = fmaxf(m, cm);
+  // A query that has seen no key yet (every score so far -inf: a split
+  // item past the query's causal limit, or a plan longer than the device
+  // kv_len) keeps m = -inf; exponents taken against 0 then give alpha = 0
+  // and p = 0 instead of exp2(-inf - -inf) = NaN, so its l and O stay 0.
+  const float mref = mn == -INFINITY ? 0.f : mn;
+  const float alpha = __builtin_amdgcn_exp2f(m - mref);
+  float p[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) p[i] = __builtin_amdgcn_exp2f(sv[i] - mref);
+  l = l * alpha + (((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7])));
+  m = mn;
+  u32x4_t pw;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) pw[w] = pack_bf16x2(p[2 * w], p[2 * w + 1]);
+  const bf16x8_t pf = as_bf16x8(pw);
+#pragma unroll
+  for (int mt = 0; mt < 4; ++mt) {
+    o[mt] *= alpha;
+    o[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf[mt]), pf, o[mt], 0, 0, 0);
+  }
+}
+
+// Keys past kv_len contribute P = 0; clear their V too (a lane's keys key0 .. key0 + 7) so stale or
+// uninitialised pool memory can never turn 0 * V into NaN.
+__device__ __forceinline__ void clear_tail(u32x4_t (&vf)[4], int key0, int kvl) {
+#pragma unroll
+  for (int mt = 0; mt < 4; ++mt) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const int key = key0 + 2 * w;
+      uint32_t x = vf[mt][w];
+      if (key >= kvl) x &= 0xffff0000u;
+      if (key + 1 >= kvl) x &= 0x0000ffffu;
+      vf[mt][w] = x;
+    }
+  }
+}
+
+// Q^T fragments (B operand) of tile qt: lane holds Q[q = qt*16 + n][hd = ks*32 + 8g .. +7].
+__device__ __forceinline__ void load_q(const AttnParams& P, int qs, int qc, int qt, int h, int g, int n,
+                                       bf16x8_t (&qf)[2]) {
+  const int q = qt * 16 + n;
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    u32x4_t v = {0u, 0u, 0u, 0u};
+    if (q < qc) v = load16(P.q + ((static_cast<int64_t>(qs) + q) * P.H + h) * kHeadDim + ks * 32 + 8 * g);
+    qf[ks] = as_bf16x8(v);
+  }
+}
+
+// o[mt][j] = O^T[hd = 16mt + 4g + j][q = qt*16 + n] to the output or, for a split item, to its slot.
+__device__ __forceinline__ void store_tile(const AttnParams& P, int qs, int qc, int qt, int h, int g, int n, int slot,
+                                           float m, float l, const f32x4_t (&o)[4]) {
+  const float L = sum_xor16_32(l);
+  const int q = qt * 16 + n;
+  if (q >= qc) return;
+  const int64_t row_q = (static_cast<int64_t>(qs) + q) * P.H + h;
+  if (slot < 0) {
+    // L = 0 only for a query that sees no key at all (an empty row): zeros, not NaN
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    uint16_t* op = P.out + row_q * kHeadDim + 4 * g;
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+      u32x2_t w2;
+      w2[0] = pack_bf16x2(o[mt][0] * inv, o[mt][1] * inv);
+      w2[1] = pack_bf16x2(o[mt][2] * inv, o[mt][3] * inv);
+      *reinterpret_cast<u32x2_t*>(op + 16 * mt) = w2;
+    }
+  } else if (slot < P.n_slots) {
+    const int64_t prow = (static_cast<int64_t>(slot) * P.bl + q) * P.H + h;
+    float* pp = P.part_o + prow * kHeadDim + 4 * g;
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) *reinterpret_cast<f32x4_t*>(pp + 16 * mt) = o[mt];
+    if (g == 0) {
+      P.part_ml[prow * 2] = m;
+      P.part_ml[prow * 2 + 1] = L;
+    }
+  }
+}
+
+// The row's page ids, 64 at a time: lane i holds the page of table column
+// base + i (clamped), and a chunk picks its two with readlane, so the
+// K/V loads never wait on a page-table load inside the loop.
+struct PageRow {
+  const int32_t* tab;
+  int last_page, max_page, lane, base, v;
+  __device__ __forceinline__ PageRow(const AttnParams& P, int r, int kvl, int kb, int lane_)
+      : tab(P.table + static_cast<int64_t>(r) * P.table_stride),
+        // reads stay inside the row even if kv_len exceeds what the table maps
+        last_page(min((kvl + kPageSize - 1) / kPageSize, P.table_cols) - 1),
+        max_page(static_cast<int>(min(P.n_pages - 1, int64_t{0x7fffffff}))), lane(lane_) {
+    load(min(kb / kPageSize, last_page));
+  }
+  __device__ __forceinline__ void load(int b) {
+    base = b;
+    v = tab[min(base + lane, last_page)];
+    asm volatile("" ::"v"(v));  // complete here: later uses wait on no load
+  }
+  __device__ __forceinline__ int operator()(int pi) {
+    pi = min(pi, last_page);
+    if (pi - base >= 64) load(pi);  // uniform: pi is the same for the wave
+    return min(max(__builtin_amdgcn_readlane(v, pi - base), 0), max_page);  // a bad table entry cannot fault
+  }
+};
+
+// Registers, measured: three and four tiles (blocks of 33-64 queries, the 64-token
+// prefill chunks) are held to two waves per SIMD -- without the bound the compiler
+// takes 222 VGPRs + 64 AGPRs for four tiles, one wave per SIMD (prefill 294 -> 280
+// ms).  One and two tiles are left at the compiler's choice: with the bound and two
+// chunks a turn a wave needs fewer instructions, but its page streams come faster
+// than HBM serves them in order (512 rows x 32: 149 -> 157 us).
 template <int NQT>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(NQT >= 3 ? 2 : 1))) void
 attn_paged_kernel(const AttnParams P) {
@@ -129,18 +258,9 @@ attn_paged_kernel(const AttnParams P) {
   const int2 rq = row_queries(P.q_start, P.n_q, r, bl);
   const int qs = rq.x, qc = rq.y;  // the row's first query row and query count
 
-  // Q^T fragments (B operand): lane holds Q[q = qt*16 + n][hd = ks*32 + 8g .. +7].
   bf16x8_t qf[NQT][2];
 #pragma unroll
-  for (int qt = 0; qt < NQT; ++qt) {
-    const int q = qt * 16 + n;
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      u32x4_t v = {0u, 0u, 0u, 0u};
-      if (q < qc) v = load16(P.q + ((static_cast<int64_t>(qs) + q) * H + h) * kHeadDim + ks * 32 + 8 * g);
-      qf[qt][ks] = as_bf16x8(v);
-    }
-  }
+  for (int qt = 0; qt < NQT; ++qt) load_q(P, qs, qc, qt, h, g, n, qf[qt]);
 
   f32x4_t o[NQT][4];
   float m[NQT], l[NQT];
@@ -152,33 +272,16 @@ attn_paged_kernel(const AttnParams P) {
     for (int mt = 0; mt < 4; ++mt) o[qt][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
 
-  const int32_t* tab = P.table + static_cast<int64_t>(r) * P.table_stride;
-  // Page-table reads stay inside the row even if kv_len exceeds what the table maps.
-  const int last_page = min((kvl + kPageSize - 1) / kPageSize, P.table_cols) - 1;
+  PageRow page_of(P, r, kvl, kb, lane);
   // Key served by row n of S^T tile t: 8*(n/4) + 4t + n%4, so that lane group g
   // ends up holding keys 8g .. 8g+7 of the chunk.
   const int key_t0 = 8 * (n >> 2) + (n & 3);
 
-  // The row's page ids, 64 at a time: lane i holds the page of table column
-  // tab_base + i (clamped), and a chunk picks its two with readlane, so the
-  // K/V loads never wait on a page-table load inside the loop.
-  int tab_base = -1;
-  int tabv = 0;
-  auto page_of = [&](int pi) -> int64_t {
-    pi = min(pi, last_page);
-    if (pi - tab_base >= 64 || tab_base < 0) {  // uniform: pi is the same for the wave
-      tab_base = pi;
-      tabv = tab[min(tab_base + lane, last_page)];
-    }
-    const int64_t pg = __builtin_amdgcn_readlane(tabv, pi - tab_base);
-    return min(max(pg, int64_t{0}), P.n_pages - 1);  // a bad table entry cannot fault
-  };
   // K fragments (A operand of S^T): tile t row n -> key key_t0 + 4t.
   // V^T fragments (A operand of O^T): row hd = 16mt + n, keys 8g .. 8g+7.
   auto load_chunk = [&](int k0, u32x4_t (&kf)[2][2], u32x4_t (&vf)[4]) {
     const int pi0 = k0 / kPageSize;
-    const int64_t p0 = page_of(pi0);
-    const int64_t p1 = page_of(pi0 + 1);
+    const int64_t p0 = page_of(pi0), p1 = page_of(pi0 + 1);
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int key = key_t0 + 4 * t;
@@ -203,79 +306,16 @@ attn_paged_kernel(const AttnParams P) {
   for (int t = 0; t < 2; ++t) asm volatile("" ::"v"(kf[t][0]), "v"(kf[t][1]));
 #pragma unroll
   for (int mt = 0; mt < 4; ++mt) asm volatile("" ::"v"(vf[mt]));
+  const int diag0 = kvl - qc;  // causal: query q may see keys <= diag0 + q
   for (int k0 = kb; k0 < ke; k0 += kChunk) {
     if (k0 + kChunk < ke) load_chunk(k0 + kChunk, kn, vn);
     const bool tail = k0 + kChunk > kvl;
-    const int diag0 = kvl - qc;  // causal: query q may see keys <= diag0 + q
     const bool mask_chunk = tail || (P.causal && k0 + kChunk > diag0 + 1);
-    if (tail) {
-      // Keys past kv_len contribute P = 0; clear their V too so stale or
-      // uninitialised pool memory can never turn 0 * V into NaN.
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt) {
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          const int key = k0 + 8 * g + 2 * w;
-          uint32_t x = vf[mt][w];
-          if (key >= kvl) x &= 0xffff0000u;
-          if (key + 1 >= kvl) x &= 0x0000ffffu;
-          vf[mt][w] = x;
-        }
-      }
-    }
-
+    if (tail) clear_tail(vf, k0 + 8 * g, kvl);
 #pragma unroll
     for (int qt = 0; qt < NQT; ++qt) {
-      f32x4_t s[2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kf[t][0]), qf[qt][0], f32x4_t{0.f, 0.f, 0.f, 0.f},
-                                                       0, 0, 0);
-        s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kf[t][1]), qf[qt][1], s[t], 0, 0, 0);
-      }
-      // s[t][j] = S[q = n][key 8g + 4t + j]
-      float sv[8];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float x = s[t][j] * P.scale_log2;
-          if (mask_chunk) {
-            const int key = k0 + 8 * g + 4 * t + j;
-            if (key >= kvl || (P.causal && key > diag0 + qt * 16 + n)) x = -INFINITY;
-          }
-          sv[4 * t + j] = x;
-        }
-      }
-      float cm = sv[0];
-#pragma unroll
-      for (int i = 1; i < 8; ++i) cm = fmaxf(cm, sv[i]);
-      cm = max_xor16_32(cm);
-      const float mn = fmaxf(m[qt], cm);
-      // A query that has seen no key yet (every score so far -inf: a split
-      // item past the query's causal limit, or a plan longer than the device
-      // kv_len) keeps m = -inf; exponents taken against 0 then give alpha = 0
-      // and p = 0 instead of exp2(-inf - -inf) = NaN, so its l and O stay 0.
-      const float mref = mn == -INFINITY ? 0.f : mn;
-      const float alpha = __builtin_amdgcn_exp2f(m[qt] - mref);
-      float ps = 0.f;
-      float p[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        p[i] = __builtin_amdgcn_exp2f(sv[i] - mref);
-        ps += p[i];
-      }
-      l[qt] = l[qt] * alpha + ps;
-      m[qt] = mn;
-      u32x4_t pw;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) pw[w] = pack_bf16x2(p[2 * w], p[2 * w + 1]);
-      const bf16x8_t pf = as_bf16x8(pw);
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt) {
-        o[qt][mt] *= alpha;
-        o[qt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf[mt]), pf, o[qt][mt], 0, 0, 0);
-      }
+      const int klim = P.causal ? min(kvl, diag0 + qt * 16 + n + 1) : kvl;
+      attn_chunk(qf[qt], kf, vf, P.scale_log2, mask_chunk, k0 + 8 * g, klim, m[qt], l[qt], o[qt]);
     }
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -285,36 +325,141 @@ attn_paged_kernel(const AttnParams P) {
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) vf[mt] = vn[mt];
   }
+#pragma unroll
+  for (int qt = 0; qt < NQT; ++qt) store_tile(P, qs, qc, qt, h, g, n, slot, m[qt], l[qt], o[qt]);
+}
 
-  // o[qt][mt][j] = O^T[hd = 16mt + 4g + j][q = qt*16 + n]
-#pragma unroll
-  for (int qt = 0; qt < NQT; ++qt) {
-    const float L = sum_xor16_32(l[qt]);
-    const int q = qt * 16 + n;
-    if (q >= qc) continue;
-    const int64_t row_q = (static_cast<int64_t>(qs) + q) * H + h;
-    if (slot < 0) {
-      // L = 0 only for a query that sees no key at all (an empty row): zeros, not NaN
-      const float inv = L > 0.f ? 1.f / L : 0.f;
-      uint16_t* op = P.out + row_q * kHeadDim + 4 * g;
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt) {
-        u32x2_t w2;
-        w2[0] = pack_bf16x2(o[qt][mt][0] * inv, o[qt][mt][1] * inv);
-        w2[1] = pack_bf16x2(o[qt][mt][2] * inv, o[qt][mt][3] * inv);
-        *reinterpret_cast<u32x2_t*>(op + 16 * mt) = w2;
-      }
-    } else if (slot < P.n_slots) {
-      const int64_t prow = (static_cast<int64_t>(slot) * bl + q) * H + h;
-      float* pp = P.part_o + prow * kHeadDim + 4 * g;
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt) *reinterpret_cast<f32x4_t*>(pp + 16 * mt) = o[qt][mt];
-      if (g == 0) {
-        P.part_ml[prow * 2] = m[qt];
-        P.part_ml[prow * 2 + 1] = L;
-      }
+// Wait until at most `later` (<= MAX, the same in every wave) chunks of LPC loads are in flight and this
+// wave's LDS reads are done; then the workgroup barrier.
+template <int MAX, int LPC, bool BARRIER>
+__device__ __forceinline__ void ring_wait(int later) {
+  if constexpr (MAX > 0) {
+    if (later < MAX) {
+      ring_wait<MAX - 1, LPC, BARRIER>(later);
+      return;
     }
   }
+  if constexpr (BARRIER) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(MAX * LPC) : "memory");
+  } else {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(MAX * LPC) : "memory");
+  }
+}
+
+// Few rows: a workgroup serves one head of an item, one wave per 16-query tile,
+// and K/V chunks come through an LDS ring (8 KB each) by direct loads, so a row's
+// chunks do not wait a memory latency each and the tiles of a block run side by
+// side.  What bounds it is one wave's issue of a chunk's ~200 instructions.
+// Every query takes its keys in the order and with the operations of
+// attn_paged_kernel: its result does not depend on which kernel runs it.
+// (Splitting a head's keys over eight waves that merge in LDS measured 8.7 us
+// against 10.0 at 2 rows x 32 queries, but its sums depend on the split.)
+//
+// LDS: K rows of 128 bytes, 16-byte chunk c of key k in slot c ^ (2 (k / 8) + (k / 2 & 1)); V^T pages of
+// 64 x 32 bytes, the halves swapped where hd & 8: the 16 lanes of a fragment read fill 16 distinct slots.
+constexpr int kRing = 3;  // chunks; 4 and 8 measured the same for few rows, slower for many (fewer workgroups per CU)
+constexpr int kRingStage = 2 * kChunk * kHeadDim * 2;
+
+template <int NQT>
+__global__ __launch_bounds__(64 * (NQT == 3 ? 4 : NQT)) __attribute__((amdgpu_waves_per_eu(2))) void  // 2: MFMAs on VGPRs
+attn_ring_kernel(const AttnParams P) {
+  constexpr int NW = NQT == 3 ? 4 : NQT, LPC = 8 / NW, NS = kRing, kStage = kRingStage;
+  extern __shared__ __attribute__((aligned(16))) char ring[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int item = static_cast<int>(blockIdx.x) / P.H;
+  const int h = static_cast<int>(blockIdx.x) - item * P.H;
+  if (P.counts != nullptr && item >= P.counts[0]) return;
+  const int4 it = reinterpret_cast<const int4*>(P.work)[item];
+  const int r = it.x, kb = it.y, ke = it.z, slot = it.w;
+  const int kvl = P.kv_len[r];
+  const int g = lane >> 4, n = lane & 15;
+  const int2 rq = row_queries(P.q_start, P.n_q, r, P.bl);
+  const int qs = rq.x, qc = rq.y;
+  bf16x8_t qf[2];
+  load_q(P, qs, qc, wave, h, g, n, qf);
+  PageRow page_of(P, r, kvl, kb, lane);
+  const int n_ch = (ke - kb + kChunk - 1) / kChunk;
+
+  // load j of a chunk (j = 0 .. 3: K keys 8j .. 8j+7; 4 .. 7: half of a V^T page), 1 KB each
+  uint32_t ofs[LPC], sofs[LPC];
+#pragma unroll
+  for (int q = 0; q < LPC; ++q) {
+    const int j = wave * LPC + q;
+    ofs[q] = j < 4 ? (lane >> 3) * 128 + 16 * ((lane & 7) ^ (2 * j + (lane >> 4 & 1)))
+                   : (lane >> 1) * 32 + 16 * ((lane & 1) ^ (lane >> 4 & 1));
+    sofs[q] = static_cast<uint32_t>(kv_plane_offset(0, j >> 2, h, P.H) * 2 + (j & 1) * 1024);
+  }
+  auto issue = [&](int c, int st) {
+    const int pi = (kb + c * kChunk) / kPageSize;
+    const __amdgpu_buffer_rsrc_t r0 = buffer_from(P.pool + kv_plane_offset(page_of(pi), 0, 0, P.H));
+    const __amdgpu_buffer_rsrc_t r1 = buffer_from(P.pool + kv_plane_offset(page_of(pi + 1), 0, 0, P.H));
+#pragma unroll
+    for (int q = 0; q < LPC; ++q) {
+      const int j = wave * LPC + q;
+      load_lds16((j & 2) ? r1 : r0, ofs[q], sofs[q], ring + st * kStage + j * 1024);
+    }
+  };
+  const int key_t0 = 8 * (n >> 2) + (n & 3);
+  const int k_sw = 2 * (n >> 2) + ((n >> 1) & 1);
+  auto read = [&](int st, u32x4_t (&kf)[2][2], u32x4_t (&vf)[4]) {
+    const char* s = ring + st * kStage;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+        kf[t][ks] = *reinterpret_cast<const u32x4_t*>(s + (key_t0 + 4 * t) * 128 + ((4 * ks + g) ^ k_sw) * 16);
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt)
+      vf[mt] = *reinterpret_cast<const u32x4_t*>(s + 4096 + (g >> 1) * 2048 + (16 * mt + n) * 32 + ((g & 1) ^ (n >> 3)) * 16);
+  };
+
+  f32x4_t o[4];
+#pragma unroll
+  for (int mt = 0; mt < 4; ++mt) o[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  asm volatile("" ::"v"(qf[0]), "v"(qf[1]));  // complete before the ring's loads are counted
+  for (int c = 0; c < NS && c < n_ch; ++c) issue(c, c);
+  u32x4_t kf[2][2], vf[4], kn[2][2], vn[4];
+  const bool computes = NQT != 3 || wave < 3;
+  if (n_ch > 0) {
+    ring_wait<NS - 1, LPC, (NW > 1)>(min(NS - 1, n_ch - 1));
+    read(0, kf, vf);
+  }
+  const int diag0 = kvl - qc;  // causal: query q may see keys <= diag0 + q
+  const int klim = P.causal ? min(kvl, diag0 + wave * 16 + n + 1) : kvl;
+  int st = 0;
+  auto step = [&](int c, bool more, u32x4_t (&kf)[2][2], u32x4_t (&vf)[4], u32x4_t (&kn)[2][2], u32x4_t (&vn)[4]) {
+    const int k0 = kb + c * kChunk;
+    const int nst = st + 1 == NS ? 0 : st + 1;
+    if (more) {
+      // chunk c + 1 has landed and every wave has read chunk c: its slot takes chunk c + NS
+      ring_wait<NS - 2, LPC, (NW > 1)>(min(NS - 2, n_ch - 2 - c));
+      if (c + NS < n_ch) issue(c + NS, st);
+      read(nst, kn, vn);
+    }
+    if (computes) {
+      const bool tail = k0 + kChunk > kvl;
+      if (tail) clear_tail(vf, k0 + 8 * g, kvl);
+      attn_chunk(qf, kf, vf, P.scale_log2, tail || (P.causal && k0 + kChunk > diag0 + 1), k0 + 8 * g, klim, m, l, o);
+    }
+    st = nst;
+  };
+  // Two chunks a turn: the fragment sets swap without copies.  Nothing in the loop
+  // is conditional: past a conditional read the compiler's waits would cover the
+  // chunk just requested.
+  int c = 0;
+  for (; c + 2 < n_ch; c += 2) {
+    step(c, true, kf, vf, kn, vn);
+    step(c + 1, true, kn, vn, kf, vf);
+  }
+  if (c + 1 < n_ch) {
+    step(c, true, kf, vf, kn, vn);
+    step(c + 1, false, kn, vn, kf, vf);
+  } else if (c < n_ch) {
+    step(c, false, kf, vf, kn, vn);
+  }
+  if (computes) store_tile(P, qs, qc, wave, h, g, n, slot, m, l, o);
 }
 
 struct MergeParams {
@@ -497,6 +642,32 @@ extern "C" int yapd_attn_plan(const int32_t* kv_len, int rows, int target_items,
 }
 
 namespace yapd {
+namespace {
+
+// The ring kernel while its head-wide workgroups and their waves leave room on
+// the chip (96 rows of 16 heads); more rows keep enough page streams in flight
+// with four heads to a workgroup.  Measured (us per launch, paged -> ring;
+// bit-identical): blocks of 32 on 182-632 keys, 2 rows 17.3 -> 10.0, 32 24.7 ->
+// 16.3, 96 40.4 -> 35.0, 128 45.1 -> 44.8, 256 84.0 -> 88.3; causal segments of 64
+// on <= 300 keys, 2 18.2 -> 8.7, 32 20.3 -> 11.9, 96 26.4 -> 24.1; blocks of 16 on
+// 64-2048 keys, 8 rows 31.6 -> 21.3, 96 87.5 -> 84.1, 256 211 -> 221.  By the rows, not the work items, whose count a captured launch
+// does not know.
+// LDS asked for only to hold attn_paged_kernel to two workgroups per CU: three
+// (one-tile blocks would fit them) are more scattered page streams at once, 256
+// rows x 16 on 116-317 keys 45.1 against 43.4 us, x 8 on 100-600 53.5 against 51.9.
+constexpr int kPagedLds = 64 * 1024;
+
+template <int NQT>
+void launch_paged(const AttnParams& P, int n_work, hipStream_t st) {
+  if (static_cast<int64_t>(P.rows) * P.H <= 1536) {
+    constexpr int NW = NQT == 3 ? 4 : NQT;
+    hipLaunchKernelGGL(attn_ring_kernel<NQT>, dim3(n_work * P.H), dim3(64 * NW), kRing * kRingStage, st, P);
+  } else {
+    hipLaunchKernelGGL(attn_paged_kernel<NQT>, dim3(n_work * (P.H / kWaves)), dim3(64 * kWaves), kPagedLds, st, P);
+  }
+}
+
+}  // namespace
 
 int attn_checks(const void* q, const void* kv_pool, int64_t n_pages, const int32_t* page_table, int table_stride,
                 int table_cols, const int32_t* kv_len, int rows, int bl, int n_heads, const int32_t* work, int n_work,
@@ -538,12 +709,11 @@ int attn_launch(const void* q, const void* kv_pool, int64_t n_pages, const int32
   P.q_start = q_start;
   P.n_q = n_q;
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  const dim3 grid(n_work * (n_heads / yapd::kWaves)), block(64 * yapd::kWaves);
   switch ((bl + 15) / 16) {
-    case 1: hipLaunchKernelGGL(yapd::attn_paged_kernel<1>, grid, block, 0, st, P); break;
-    case 2: hipLaunchKernelGGL(yapd::attn_paged_kernel<2>, grid, block, 0, st, P); break;
-    case 3: hipLaunchKernelGGL(yapd::attn_paged_kernel<3>, grid, block, 0, st, P); break;
-    default: hipLaunchKernelGGL(yapd::attn_paged_kernel<4>, grid, block, 0, st, P); break;
+    case 1: yapd::launch_paged<1>(P, n_work, st); break;
+    case 2: yapd::launch_paged<2>(P, n_work, st); break;
+    case 3: yapd::launch_paged<3>(P, n_work, st); break;
+    default: yapd::launch_paged<4>(P, n_work, st); break;
   }
   YAPD_LAUNCH_CHECK("attn_paged_kernel launch");
   if (n_merge > 0) {
