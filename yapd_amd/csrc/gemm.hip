@@ -938,18 +938,43 @@ __device__ __forceinline__ void sk_rows(const GemmParams& p, int m0, int wm, int
   }
 }
 
+__device__ __forceinline__ bool c_vec4(const GemmParams& p) {
+  return p.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(p.C) & 7u) == 0;
+}
+
+// This lane's residual values (kEpiResidual), requested before the main loop:
+// behind it they would cost a memory latency each, as every store to C could
+// alias the next load (down, M = 1630: 25.1 -> 22.4 us).
+template <class T>
+__device__ __forceinline__ void sk_residual(const GemmParams& p, int m0, int bx, int wm, int wn, int tok, int sub,
+                                            u32x2_t (&res)[T::TM][T::TN]) {
+  const bool vec_ok = c_vec4(p);
+#pragma unroll
+  for (int i = 0; i < T::TM; ++i) {
+    const int m = m0 + (wm * T::TM + i) * 16 + tok;
+#pragma unroll
+    for (int j = 0; j < T::TN; ++j) {
+      const int n = bx * T::BN + (wn * T::TN + j) * 16 + sub;
+      res[i][j] = u32x2_t{0u, 0u};
+      if (vec_ok && m < p.M && n + 4 <= p.N)
+        res[i][j] = *reinterpret_cast<const u32x2_t*>(p.C + static_cast<int64_t>(m) * p.ldc + n);
+    }
+  }
+}
+
 // Epilogues of the 16 x 16 sub-tile kernels, from registers.
 template <class T, int EPI>
 __device__ __forceinline__ void sk_finish(const GemmParams& p, const f32x4_t (&acc)[T::TM][T::TN],
-                                          const int (&pos)[T::TM], const int (&prow)[T::TM], int m0, int bx, int wm,
-                                          int wn, int tok, int sub) {
+                                          const int (&pos)[T::TM], const int (&prow)[T::TM],
+                                          const u32x2_t (&res)[T::TM][T::TN], int m0, int bx, int wm, int wn, int tok,
+                                          int sub) {
   constexpr bool kPair = EPI == kEpiQkv || EPI == kEpiSwiglu;
 #pragma unroll
   for (int i = 0; i < T::TM; ++i) {
     const int m = m0 + (wm * T::TM + i) * 16 + tok;
     if (m >= p.M) continue;
     if constexpr (!kPair) {
-      const bool vec_ok = (p.ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(p.C) & 7u) == 0);
+      const bool vec_ok = c_vec4(p);
       uint16_t* const row = p.C + static_cast<int64_t>(m) * p.ldc;
 #pragma unroll
       for (int j = 0; j < T::TN; ++j) {
@@ -957,10 +982,9 @@ __device__ __forceinline__ void sk_finish(const GemmParams& p, const f32x4_t (&a
         u32x2_t v = {pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3])};
         if (vec_ok && n + 4 <= p.N) {
           if constexpr (EPI == kEpiResidual) {
-            const u32x2_t r = *reinterpret_cast<const u32x2_t*>(row + n);
 #pragma unroll
             for (int w = 0; w < 2; ++w)
-              v[w] = pack_bf16x2(bf16lo(r[w]) + bf16lo(v[w]), bf16hi(r[w]) + bf16hi(v[w]));
+              v[w] = pack_bf16x2(bf16lo(res[i][j][w]) + bf16lo(v[w]), bf16hi(res[i][j][w]) + bf16hi(v[w]));
           }
           *reinterpret_cast<u32x2_t*>(row + n) = v;
         } else {
@@ -974,7 +998,7 @@ __device__ __forceinline__ void sk_finish(const GemmParams& p, const f32x4_t (&a
         }
       }
     } else if constexpr (EPI == kEpiSwiglu) {
-      const bool vec_ok = (p.ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(p.C) & 7u) == 0);
+      const bool vec_ok = c_vec4(p);
       uint16_t* const row = p.C + static_cast<int64_t>(m) * p.ldc;
 #pragma unroll
       for (int j = 0; j < T::TN; j += 2) {
@@ -1076,6 +1100,9 @@ __global__ __launch_bounds__(T::THREADS) void gemm_sk_kernel(const GemmParams p)
   const int tok = lane & 15, sub = 4 * (lane >> 4);
   int pos[T::TM], prow[T::TM];
   if constexpr (EPI == kEpiQkv) sk_rows<T>(p, m0, wm, tok, pos, prow);
+  u32x2_t res[T::TM][T::TN];
+  if constexpr (EPI == kEpiResidual)
+    if (wave < T::WM * T::WN) sk_residual<T>(p, m0, bx, wm, wn, tok, sub, res);
 #pragma unroll
   for (int s = 0; s + 1 < T::NS; ++s)
     if (s < st_n) issue(s, s);
@@ -1149,7 +1176,7 @@ __global__ __launch_bounds__(T::THREADS) void gemm_sk_kernel(const GemmParams p)
   while (st + T::NS - 1 < st_n) stage(std::integral_constant<int, 0>{});
   while (st + 1 < st_n) stage(std::integral_constant<int, 1>{});
   stage(std::integral_constant<int, 2>{});
-  sk_finish<T, EPI>(p, acc, pos, prow, m0, bx, wm, wn, tok, sub);
+  sk_finish<T, EPI>(p, acc, pos, prow, res, m0, bx, wm, wn, tok, sub);
 }
 
 // Affine-quantised W on the same tiles: A as above; W's codes come to LDS by
@@ -1315,6 +1342,9 @@ __global__ __launch_bounds__(Q::T::THREADS) void gemm_skq_kernel(const GemmParam
   const int tok = lane & 15, sub = 4 * (lane >> 4);
   int pos[T::TM], prow[T::TM];
   if constexpr (EPI == kEpiQkv) sk_rows<T>(p, m0, wm, tok, pos, prow);
+  u32x2_t res[T::TM][T::TN];
+  if constexpr (EPI == kEpiResidual)
+    if (wave < T::WM * T::WN) sk_residual<T>(p, m0, bx, wm, wn, tok, sub, res);
 
   // Prologue: codes 0, then steps 0 .. NA - 2 (A i, codes i + 1), A of step NA - 1 and, once the
   // slot of codes 0 is free, its codes.
@@ -1437,7 +1467,7 @@ __global__ __launch_bounds__(Q::T::THREADS) void gemm_skq_kernel(const GemmParam
   while (st + NA < st_n) stage(std::integral_constant<int, 0>{});
   while (st + 1 < st_n) stage(std::integral_constant<int, 1>{});
   stage(std::integral_constant<int, 2>{});
-  sk_finish<T, EPI>(p, acc, pos, prow, m0, bx, wm, wn, tok, sub);
+  sk_finish<T, EPI>(p, acc, pos, prow, res, m0, bx, wm, wn, tok, sub);
 }
 
 // Affine-quantised W on the direct-load layout: A moves global -> LDS by
