@@ -139,6 +139,9 @@ def check(rc: int) -> None:
 
 
 def stream_ptr(device: torch.device) -> int:
+    # the raw handle: building a torch.cuda.Stream object costs more than the launch it is for
+    if device.index is not None:
+        return torch._C._cuda_getCurrentRawStream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 
@@ -153,11 +156,13 @@ def require(cond: bool, msg: str) -> None:
 
 def require_cuda(t: torch.Tensor, name: str, dtype: torch.dtype, device: torch.device,
                  contiguous: bool = True) -> None:
+    # one test on the way of every call; the messages are formatted only for a tensor that fails it
+    if t.is_cuda and t.dtype == dtype and t.device == device and (not contiguous or t.is_contiguous()):
+        return
     require(t.is_cuda, f"{name} must be a GPU tensor")
     require(t.device == device, f"{name} is on {t.device}, expected {device}")
     require(t.dtype == dtype, f"{name} must be {dtype}, got {t.dtype}")
-    if contiguous:
-        require(t.is_contiguous(), f"{name} must be contiguous")
+    require(t.is_contiguous(), f"{name} must be contiguous")
 
 
 # --------------------------------------------------------------------------- #
@@ -184,12 +189,14 @@ def score_cfg_pmi_unmask(
     require(logits.dim() == 3 and logits.stride(2) == 1, "logits must be [rows, bl, V] with unit last stride")
     rows, bl, V = logits.shape
     last_row = cond_row0 + (n_pairs - 1) * pair_row_step + max(0, null_row_offset or 0)
-    require(0 <= cond_row0 and last_row < rows, f"pair layout reaches row {last_row} of {rows}")
+    if not (0 <= cond_row0 and last_row < rows):
+        raise ValueError(f"pair layout reaches row {last_row} of {rows}")
     require(null_row_offset is None or cond_row0 + null_row_offset >= 0, "null rows out of range")
     require_cuda(log_prior, "log_prior", torch.float32, dev)
     require(log_prior.numel() == V, "log_prior must have V entries")
     require_cuda(xt_blk, "xt_blk", torch.int64, dev)
-    require(tuple(xt_blk.shape) == (n_pairs, bl), f"xt_blk must be [{n_pairs}, {bl}]")
+    if not (tuple(xt_blk.shape) == (n_pairs, bl)):
+        raise ValueError(f"xt_blk must be [{n_pairs}, {bl}]")
     require_cuda(k_step, "k_step", torch.int64, dev)
     require(k_step.numel() == n_pairs, "k_step must have n_pairs entries")
     require_cuda(sched, "sched", torch.int32, dev)
@@ -203,7 +210,8 @@ def score_cfg_pmi_unmask(
                             ("n_mask_after", torch.int32, (n_pairs,)), ("hit_eos", torch.uint8, (n_pairs,))):
         t = out[name]
         require_cuda(t, name, dt, dev)
-        require(tuple(t.shape) == shape, f"{name} must be {shape}")
+        if not (tuple(t.shape) == shape):
+            raise ValueError(f"{name} must be {shape}")
     check(lib.yapd_score_cfg_pmi_unmask(
         logits.data_ptr(), logits.stride(0), logits.stride(1), n_pairs, bl, V,
         cond_row0, pair_row_step, 0 if null_row_offset is None else 1, null_row_offset or 0,
@@ -326,7 +334,8 @@ def kv_gather(pool: torch.Tensor, table_row: torch.Tensor, kv_len: int):
 
 def _mat(t: torch.Tensor, name: str, dev) -> None:
     require_cuda(t, name, torch.bfloat16, dev, contiguous=False)
-    require(t.dim() == 2 and t.stride(1) == 1, f"{name} must be a 2-D row-major view")
+    if not (t.dim() == 2 and t.stride(1) == 1):
+        raise ValueError(f"{name} must be a 2-D row-major view")
 
 
 def gemm_bf16(A: torch.Tensor, W: torch.Tensor, out: torch.Tensor) -> None:
@@ -511,12 +520,14 @@ def tick_update(*, xt: torch.Tensor, xt_blk: torch.Tensor, xt_new: torch.Tensor,
     D = hidden.shape[-1]
     for name, t in (("xt_blk", xt_blk), ("xt_new", xt_new), ("xt_final", xt_final)):
         require_cuda(t, name, torch.int64, dev)
-        require(tuple(t.shape) == (S, bl), f"{name} must be [slots, bl]")
+        if not (tuple(t.shape) == (S, bl)):
+            raise ValueError(f"{name} must be [slots, bl]")
     require_cuda(xt, "xt", torch.int64, dev, contiguous=False)
     require(xt.dim() == 2 and xt.stride(1) == 1 and xt.shape[0] >= S, "xt must be [slots, n_max] row-major")
     for name, t in (("k_step", k_step), ("cache_len", cache_len), ("blk_start", blk_start), ("n_speech", n_speech)):
         require_cuda(t, name, torch.int64, dev)
-        require(t.numel() >= S, f"{name} needs one entry per slot")
+        if not (t.numel() >= S):
+            raise ValueError(f"{name} needs one entry per slot")
     require_cuda(is_commit, "is_commit", torch.uint8, dev)
     require(is_commit.numel() >= S, "is_commit needs one entry per slot")
     require_cuda(hidden, "hidden", torch.bfloat16, dev)
@@ -551,7 +562,8 @@ def voc_stitch(wav: torch.Tensor, jobs: torch.Tensor, fade_in: torch.Tensor, fad
     require_cuda(wav, "wav", torch.float32, dev, contiguous=False)
     require(wav.dim() == 2 and wav.stride(1) == 1, "wav must be [rows, samples] with unit last stride")
     require_cuda(jobs, "jobs", torch.int32, dev)
-    require(jobs.dim() == 2 and jobs.shape[1] == STITCH_JOB_INTS, f"jobs must be [n, {STITCH_JOB_INTS}]")
+    if not (jobs.dim() == 2 and jobs.shape[1] == STITCH_JOB_INTS):
+        raise ValueError(f"jobs must be [n, {STITCH_JOB_INTS}]")
     fade = fade_in.numel()
     for t, name in ((fade_in, "fade_in"), (fade_out, "fade_out"), (trim, "trim")):
         require_cuda(t, name, torch.float32, dev)
@@ -559,7 +571,8 @@ def voc_stitch(wav: torch.Tensor, jobs: torch.Tensor, fade_in: torch.Tensor, fad
     for t, name in ((tails_in, "tails_in"), (tails_out, "tails_out")):
         if t is not None:
             require_cuda(t, name, torch.float32, dev)
-            require(t.dim() == 2 and t.shape[1] == fade, f"{name} must be [n, {fade}]")
+            if not (t.dim() == 2 and t.shape[1] == fade):
+                raise ValueError(f"{name} must be [n, {fade}]")
     require_cuda(pcm, "pcm", torch.int16, dev)
     n_in = 0 if tails_in is None else tails_in.shape[0]
     n_out = 0 if tails_out is None else tails_out.shape[0]

@@ -97,6 +97,7 @@ class AttnPlan:
                  target_items: int = 192, min_split_keys: int = 1024):
         work, merge, n_slots = kernels.attn_plan(kv_len, target_items=target_items, min_split_keys=min_split_keys)
         self.kv_len_host = [int(x) for x in kv_len]
+        self._max_kv_len = max(self.kv_len_host)  # of the planned lengths, which do not change
         self.work = to_device_async(work, torch.int32, device)
         self.merge = to_device_async(merge, torch.int32, device) if merge.shape[0] else None
         self.n_slots = n_slots
@@ -109,7 +110,7 @@ class AttnPlan:
 
     def run(self, q: torch.Tensor, pool: torch.Tensor, table: torch.Tensor, out: torch.Tensor,
             scale: float, causal: bool = False) -> None:
-        kernels.require(max(self.kv_len_host) <= table.shape[1] * PAGE_SIZE,
+        kernels.require(self._max_kv_len <= table.shape[1] * PAGE_SIZE,
                         "page table maps fewer positions than kv_len")
         kernels.attn_paged_block(q, pool, table, self.kv_len, self.work, self.merge, self.part_o, self.part_ml,
                                  out, scale, causal=causal)

@@ -55,7 +55,8 @@ def _check_codes(packed: torch.Tensor, scales: torch.Tensor, biases: torch.Tenso
     kernels.require(packed.shape[1] * 32 // bits == K, "packed width does not match K")
     for name, t in (("scales", scales), ("biases", biases)):
         kernels.require_cuda(t, name, torch.float16, dev)
-        kernels.require(tuple(t.shape) == (N, K // GROUP), f"{name} must be [N, K/64]")
+        if tuple(t.shape) != (N, K // GROUP):
+            raise ValueError(f"{name} must be [N, K/64]")
     return N
 
 
@@ -108,6 +109,8 @@ class QuantLinear:
 
     def __call__(self, x: torch.Tensor, out: Optional[torch.Tensor] = None,
                  scratch: Optional[torch.Tensor] = None) -> torch.Tensor:
+        if x.dim() == 2 and (out is None or (out.dim() == 2 and out.shape[1] == self.out_features)):
+            return qgemm_affine(x, self.packed, self.scales, self.biases, self.bits, out=out, scratch=scratch)
         lead = x.shape[:-1]
         y = qgemm_affine(x.reshape(-1, self.in_features), self.packed, self.scales, self.biases, self.bits,
                          out=None if out is None else out.view(-1, self.out_features), scratch=scratch)
