@@ -1,6 +1,6 @@
 // (c) CFG combine + prior-calibrated PMI + time-shifted-quantile unmask.
 //
-// One workgroup of 16 waves per CFG pair.  Each wave scores whole positions:
+// One workgroup of 16 waves per CFG pair (few pairs: see launch_score).  Each wave scores whole positions:
 // it streams the position's cond and null logit rows once from HBM (dword
 // loads; rows are only 4-byte aligned since V = 8194), each lane keeping a
 // running (max, sum-exp) per branch and its best guided score, then reduces
@@ -517,6 +517,63 @@ __global__ __launch_bounds__(64 * kPairWaves) void score_pair_kernel(const Score
   }
 }
 
+// Few pairs: the positions spread over workgroups of kItemWaves, each wave
+// finishing its position's token and pmi, and a second launch applies the
+// decision rule to the pair.  The same operations on the same values as
+// score_pair_kernel, so the outputs are equal bit for bit.
+constexpr int kItemWaves = 4;
+
+template <bool kHasU, bool kSample, bool kRank = false>
+__global__ __launch_bounds__(64 * kItemWaves) void score_item_kernel(const ScoreParams P) {
+  const int pair = blockIdx.y;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int pos = blockIdx.x * kItemWaves + wave;
+  __shared__ float4 s_sav[kItemWaves * (kUnroll / 2) * 64];
+  if (pos >= P.bl) return;
+  const int item = pair * P.bl + pos;
+  const ItemStats st = score_item<kHasU, kSample, kRank>(P, item, pair, pos, lane, s_sav + wave * (kUnroll / 2) * 64);
+  if (lane == 0) {
+    P.pmi[item] = item_pmi<kHasU>(P, item, pair, pos, st, P.xt_in[item]);
+    P.sampled[item] = st.x;
+  }
+}
+
+__global__ __launch_bounds__(64) void score_decide_kernel(const ScoreParams P) {
+  const int pair = blockIdx.x, lane = threadIdx.x;
+  __shared__ __align__(16) uint64_t s_ka[64];
+  __shared__ __align__(16) uint64_t s_kd[64];
+  const PairInputs in = load_pair_inputs(P, pair, lane);
+  float pmi = 0.f;
+  int64_t x = 0;
+  if (lane < P.bl) {
+    pmi = P.pmi[pair * P.bl + lane];
+    x = P.sampled[pair * P.bl + lane];
+  }
+  decide_pair(P, pair, lane, in, pmi, x, s_ka, s_kd);
+}
+
+// score_pair_kernel leaves the CUs without a pair idle and one wave takes up to
+// four positions in turn; two launches pay while pairs fill at most half of the
+// CUs and a pair has more positions than half of its waves.  Measured (us, with a
+// null row, pair kernel -> two launches): blocks of 32, 1 pair 30.7 -> 11.1, 32
+// 32.5 -> 14.4, 128 40.2 -> 32.9, 192 44.7 -> 45.2; of 16, 5 17.9 -> 11.5, 128
+// 19.9 -> 18.6, 160 21.4 -> 23.0; of 8, 5 12.0 -> 11.3 (without a null row 8.5 ->
+// 9.0), 64 13.0 -> 13.1.
+template <bool kHasU, bool kSample, bool kRank = false>
+int launch_score(const ScoreParams& P, hipStream_t st) {
+  if (P.n_pairs <= 128 && P.bl > 8) {
+    const dim3 grid((P.bl + kItemWaves - 1) / kItemWaves, P.n_pairs);
+    hipLaunchKernelGGL((score_item_kernel<kHasU, kSample, kRank>), grid, dim3(64 * kItemWaves), 0, st, P);
+    YAPD_LAUNCH_CHECK("score_item_kernel launch");
+    hipLaunchKernelGGL(score_decide_kernel, dim3(P.n_pairs), dim3(64), 0, st, P);
+    YAPD_LAUNCH_CHECK("score_decide_kernel launch");
+    return YAPD_OK;
+  }
+  hipLaunchKernelGGL((score_pair_kernel<kHasU, kSample, kRank>), dim3(P.n_pairs), dim3(64 * kPairWaves), 0, st, P);
+  YAPD_LAUNCH_CHECK("score_pair_kernel launch");
+  return YAPD_OK;
+}
+
 }  // namespace
 }  // namespace yapd
 
@@ -577,17 +634,9 @@ extern "C" int yapd_score_cfg_pmi_unmask(
   P.n_mask_after = n_mask_after_out;
   P.hit_eos = hit_eos_out;
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  const dim3 grid(n_pairs), block(64 * yapd::kPairWaves);
-  if (has_uncond && temperature > 0.f)
-    hipLaunchKernelGGL((yapd::score_pair_kernel<true, true>), grid, block, 0, st, P);
-  else if (has_uncond && cfg_w > 0.f)
-    hipLaunchKernelGGL((yapd::score_pair_kernel<true, false, true>), grid, block, 0, st, P);
-  else if (has_uncond)
-    hipLaunchKernelGGL((yapd::score_pair_kernel<true, false>), grid, block, 0, st, P);
-  else if (temperature > 0.f)
-    hipLaunchKernelGGL((yapd::score_pair_kernel<false, true>), grid, block, 0, st, P);
-  else
-    hipLaunchKernelGGL((yapd::score_pair_kernel<false, false>), grid, block, 0, st, P);
-  YAPD_LAUNCH_CHECK("score_pair_kernel launch");
-  return YAPD_OK;
+  if (has_uncond && temperature > 0.f) return yapd::launch_score<true, true>(P, st);
+  if (has_uncond && cfg_w > 0.f) return yapd::launch_score<true, false, true>(P, st);
+  if (has_uncond) return yapd::launch_score<true, false>(P, st);
+  if (temperature > 0.f) return yapd::launch_score<false, true>(P, st);
+  return yapd::launch_score<false, false>(P, st);
 }
