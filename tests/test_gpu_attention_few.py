@@ -39,7 +39,7 @@ def run(dev, rows, bl, H, lens, causal=False, **plan_kw):
 
 
 @pytest.mark.parametrize("bl", [1, 16, 17, 32, 48, 64])
-@pytest.mark.parametrize("rows", [1, 3, 17, 96])  # H = 16: 96 rows are the limit
+@pytest.mark.parametrize("rows", [1, 3, 17, 64, 96])  # H = 16: 96 rows are the limit, 64 with bl > 32
 @pytest.mark.parametrize("causal", [False, True])
 def test_few_rows(dev, rows, bl, causal):
     lens = [max(bl, n) for n in ([1, 31, 32, 33, 64, 97, 129, 300, 541] * 11)[:rows]]

@@ -329,31 +329,28 @@ attn_paged_kernel(const AttnParams P) {
   for (int qt = 0; qt < NQT; ++qt) store_tile(P, qs, qc, qt, h, g, n, slot, m[qt], l[qt], o[qt]);
 }
 
-// Wait until at most `later` (<= MAX, the same in every wave) chunks of LPC loads are in flight and this
-// wave's LDS reads are done; then the workgroup barrier.
-template <int MAX, int LPC, bool BARRIER>
+// Wait until at most `later` (<= MAX) chunks of 8 loads are in flight, then the workgroup barrier.
+template <int MAX>
 __device__ __forceinline__ void ring_wait(int later) {
   if constexpr (MAX > 0) {
     if (later < MAX) {
-      ring_wait<MAX - 1, LPC, BARRIER>(later);
+      ring_wait<MAX - 1>(later);
       return;
     }
   }
-  if constexpr (BARRIER) {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(MAX * LPC) : "memory");
-  } else {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(MAX * LPC) : "memory");
-  }
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(MAX * 8) : "memory");
 }
 
 // Few rows: a workgroup serves one head of an item, one wave per 16-query tile,
-// and K/V chunks come through an LDS ring (8 KB each) by direct loads, so a row's
-// chunks do not wait a memory latency each and the tiles of a block run side by
-// side.  What bounds it is one wave's issue of a chunk's ~200 instructions.
+// and one more wave brings the K/V chunks into an LDS ring (8 KB each) by direct
+// loads, so a row's chunks do not wait a memory latency each and the tiles of a
+// block run side by side.  What bounds it is one wave's issue of a chunk's ~150
+// instructions; with the loads among them, on the same wave, ~200: 2 rows x 32
+// queries 10.0 us against 8.6, 8 rows x 16 on 64-2048 keys 21.3 against 17.6.
 // Every query takes its keys in the order and with the operations of
 // attn_paged_kernel: its result does not depend on which kernel runs it.
 // (Splitting a head's keys over eight waves that merge in LDS measured 8.7 us
-// against 10.0 at 2 rows x 32 queries, but its sums depend on the split.)
+// against 8.6 at 2 rows x 32 queries, and its sums depend on the split.)
 //
 // LDS: K rows of 128 bytes, 16-byte chunk c of key k in slot c ^ (2 (k / 8) + (k / 2 & 1)); V^T pages of
 // 64 x 32 bytes, the halves swapped where hd & 8: the 16 lanes of a fragment read fill 16 distinct slots.
@@ -361,9 +358,9 @@ constexpr int kRing = 3;  // chunks; 4 and 8 measured the same for few rows, slo
 constexpr int kRingStage = 2 * kChunk * kHeadDim * 2;
 
 template <int NQT>
-__global__ __launch_bounds__(64 * (NQT == 3 ? 4 : NQT)) __attribute__((amdgpu_waves_per_eu(2))) void  // 2: MFMAs on VGPRs
+__global__ __launch_bounds__(64 * (NQT + 1)) __attribute__((amdgpu_waves_per_eu(2))) void  // 2: MFMAs on VGPRs
 attn_ring_kernel(const AttnParams P) {
-  constexpr int NW = NQT == 3 ? 4 : NQT, LPC = 8 / NW, NS = kRing, kStage = kRingStage;
+  constexpr int NS = kRing, kStage = kRingStage;
   extern __shared__ __attribute__((aligned(16))) char ring[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -376,30 +373,41 @@ attn_ring_kernel(const AttnParams P) {
   const int g = lane >> 4, n = lane & 15;
   const int2 rq = row_queries(P.q_start, P.n_q, r, P.bl);
   const int qs = rq.x, qc = rq.y;
-  bf16x8_t qf[2];
-  load_q(P, qs, qc, wave, h, g, n, qf);
-  PageRow page_of(P, r, kvl, kb, lane);
   const int n_ch = (ke - kb + kChunk - 1) / kChunk;
 
-  // load j of a chunk (j = 0 .. 3: K keys 8j .. 8j+7; 4 .. 7: half of a V^T page), 1 KB each
-  uint32_t ofs[LPC], sofs[LPC];
+  if (wave == NQT) {
+    // load j of a chunk (j = 0 .. 3: K keys 8j .. 8j+7; 4 .. 7: half of a V^T page), 1 KB each
+    PageRow page_of(P, r, kvl, kb, lane);
+    uint32_t ofs[5];  // K rows j, then V^T
 #pragma unroll
-  for (int q = 0; q < LPC; ++q) {
-    const int j = wave * LPC + q;
-    ofs[q] = j < 4 ? (lane >> 3) * 128 + 16 * ((lane & 7) ^ (2 * j + (lane >> 4 & 1)))
-                   : (lane >> 1) * 32 + 16 * ((lane & 1) ^ (lane >> 4 & 1));
-    sofs[q] = static_cast<uint32_t>(kv_plane_offset(0, j >> 2, h, P.H) * 2 + (j & 1) * 1024);
-  }
-  auto issue = [&](int c, int st) {
-    const int pi = (kb + c * kChunk) / kPageSize;
-    const __amdgpu_buffer_rsrc_t r0 = buffer_from(P.pool + kv_plane_offset(page_of(pi), 0, 0, P.H));
-    const __amdgpu_buffer_rsrc_t r1 = buffer_from(P.pool + kv_plane_offset(page_of(pi + 1), 0, 0, P.H));
+    for (int j = 0; j < 4; ++j) ofs[j] = (lane >> 3) * 128 + 16 * ((lane & 7) ^ (2 * j + (lane >> 4 & 1)));
+    ofs[4] = (lane >> 1) * 32 + 16 * ((lane & 1) ^ (lane >> 4 & 1));
+    const uint32_t k_plane = static_cast<uint32_t>(kv_plane_offset(0, 0, h, P.H) * 2);
+    const uint32_t v_plane = static_cast<uint32_t>(kv_plane_offset(0, 1, h, P.H) * 2);
+    auto issue = [&](int c, int st) {
+      const int pi = (kb + c * kChunk) / kPageSize;
+      const __amdgpu_buffer_rsrc_t r0 = buffer_from(P.pool + kv_plane_offset(page_of(pi), 0, 0, P.H));
+      const __amdgpu_buffer_rsrc_t r1 = buffer_from(P.pool + kv_plane_offset(page_of(pi + 1), 0, 0, P.H));
 #pragma unroll
-    for (int q = 0; q < LPC; ++q) {
-      const int j = wave * LPC + q;
-      load_lds16((j & 2) ? r1 : r0, ofs[q], sofs[q], ring + st * kStage + j * 1024);
+      for (int j = 0; j < 8; ++j)
+        load_lds16((j & 2) ? r1 : r0, ofs[j < 4 ? j : 4], (j < 4 ? k_plane : v_plane) + (j & 1) * 1024,
+                   ring + st * kStage + j * 1024);
+    };
+    for (int c = 0; c < NS && c < n_ch; ++c) issue(c, c);
+    if (n_ch > 0) ring_wait<NS - 1>(min(NS - 1, n_ch - 1));
+    int st = 0;
+    for (int c = 0; c + 1 < n_ch; ++c) {
+      // chunk c + 1 has landed and every wave has read chunk c: its slot takes chunk c + NS
+      ring_wait<NS - 2>(min(NS - 2, n_ch - 2 - c));
+      if (c + NS < n_ch) issue(c + NS, st);
+      st = st + 1 == NS ? 0 : st + 1;
     }
-  };
+    return;
+  }
+  bf16x8_t qf[2];
+  load_q(P, qs, qc, wave, h, g, n, qf);
+  // this wave's LDS reads are done; the loader's chunk has landed
+  auto hand_over = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
   const int key_t0 = 8 * (n >> 2) + (n & 3);
   const int k_sw = 2 * (n >> 2) + ((n >> 1) & 1);
   auto read = [&](int st, u32x4_t (&kf)[2][2], u32x4_t (&vf)[4]) {
@@ -418,12 +426,9 @@ attn_ring_kernel(const AttnParams P) {
 #pragma unroll
   for (int mt = 0; mt < 4; ++mt) o[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
-  asm volatile("" ::"v"(qf[0]), "v"(qf[1]));  // complete before the ring's loads are counted
-  for (int c = 0; c < NS && c < n_ch; ++c) issue(c, c);
   u32x4_t kf[2][2], vf[4], kn[2][2], vn[4];
-  const bool computes = NQT != 3 || wave < 3;
   if (n_ch > 0) {
-    ring_wait<NS - 1, LPC, (NW > 1)>(min(NS - 1, n_ch - 1));
+    hand_over();
     read(0, kf, vf);
   }
   const int diag0 = kvl - qc;  // causal: query q may see keys <= diag0 + q
@@ -433,16 +438,12 @@ attn_ring_kernel(const AttnParams P) {
     const int k0 = kb + c * kChunk;
     const int nst = st + 1 == NS ? 0 : st + 1;
     if (more) {
-      // chunk c + 1 has landed and every wave has read chunk c: its slot takes chunk c + NS
-      ring_wait<NS - 2, LPC, (NW > 1)>(min(NS - 2, n_ch - 2 - c));
-      if (c + NS < n_ch) issue(c + NS, st);
+      hand_over();
       read(nst, kn, vn);
     }
-    if (computes) {
-      const bool tail = k0 + kChunk > kvl;
-      if (tail) clear_tail(vf, k0 + 8 * g, kvl);
-      attn_chunk(qf, kf, vf, P.scale_log2, tail || (P.causal && k0 + kChunk > diag0 + 1), k0 + 8 * g, klim, m, l, o);
-    }
+    const bool tail = k0 + kChunk > kvl;
+    if (tail) clear_tail(vf, k0 + 8 * g, kvl);
+    attn_chunk(qf, kf, vf, P.scale_log2, tail || (P.causal && k0 + kChunk > diag0 + 1), k0 + 8 * g, klim, m, l, o);
     st = nst;
   };
   // Two chunks a turn: the fragment sets swap without copies.  Nothing in the loop
@@ -459,7 +460,7 @@ attn_ring_kernel(const AttnParams P) {
   } else if (c < n_ch) {
     step(c, false, kf, vf, kn, vn);
   }
-  if (computes) store_tile(P, qs, qc, wave, h, g, n, slot, m, l, o);
+  store_tile(P, qs, qc, wave, h, g, n, slot, m, l, o);
 }
 
 struct MergeParams {
@@ -644,24 +645,24 @@ extern "C" int yapd_attn_plan(const int32_t* kv_len, int rows, int target_items,
 namespace yapd {
 namespace {
 
-// The ring kernel while its head-wide workgroups and their waves leave room on
-// the chip (96 rows of 16 heads); more rows keep enough page streams in flight
-// with four heads to a workgroup.  Measured (us per launch, paged -> ring;
-// bit-identical): blocks of 32 on 182-632 keys, 2 rows 17.3 -> 10.0, 32 24.7 ->
-// 16.3, 96 40.4 -> 35.0, 128 45.1 -> 44.8, 256 84.0 -> 88.3; causal segments of 64
-// on <= 300 keys, 2 18.2 -> 8.7, 32 20.3 -> 11.9, 96 26.4 -> 24.1; blocks of 16 on
-// 64-2048 keys, 8 rows 31.6 -> 21.3, 96 87.5 -> 84.1, 256 211 -> 221.  By the rows, not the work items, whose count a captured launch
-// does not know.
 // LDS asked for only to hold attn_paged_kernel to two workgroups per CU: three
 // (one-tile blocks would fit them) are more scattered page streams at once, 256
 // rows x 16 on 116-317 keys 45.1 against 43.4 us, x 8 on 100-600 53.5 against 51.9.
 constexpr int kPagedLds = 64 * 1024;
 
+// The ring kernel while its head-wide workgroups and their waves leave room on
+// the chip (96 rows of 16 heads, 64 with three or four tiles); more rows keep
+// enough page streams in flight with four heads to a workgroup.  Measured (us per
+// launch, paged -> ring; bit-identical): blocks of 32 on 182-632 keys, 2 rows 16.4
+// -> 8.6, 32 23.9 -> 15.5, 96 40.5 -> 34.4, 128 45.1 -> 45.3; causal segments of 64
+// on <= 300 keys, 2 17.3 -> 7.9, 32 19.5 -> 11.2, 64 21.2 -> 19.6, 96 25.7 -> 26.6;
+// blocks of 16 on 64-2048 keys, 8 rows 31.7 -> 17.6, 64 67.2 -> 62.9, 128 114.6 ->
+// 115.5.  By the rows, not the work items, whose count a captured launch does not
+// know.
 template <int NQT>
 void launch_paged(const AttnParams& P, int n_work, hipStream_t st) {
-  if (static_cast<int64_t>(P.rows) * P.H <= 1536) {
-    constexpr int NW = NQT == 3 ? 4 : NQT;
-    hipLaunchKernelGGL(attn_ring_kernel<NQT>, dim3(n_work * P.H), dim3(64 * NW), kRing * kRingStage, st, P);
+  if (static_cast<int64_t>(P.rows) * P.H <= (NQT >= 3 ? 1024 : 1536) && n_work <= INT32_MAX / P.H) {
+    hipLaunchKernelGGL(attn_ring_kernel<NQT>, dim3(n_work * P.H), dim3(64 * (NQT + 1)), kRing * kRingStage, st, P);
   } else {
     hipLaunchKernelGGL(attn_paged_kernel<NQT>, dim3(n_work * (P.H / kWaves)), dim3(64 * kWaves), kPagedLds, st, P);
   }
