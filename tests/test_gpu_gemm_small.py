@@ -102,3 +102,17 @@ def test_wide_row_pitch(dev):
     kernels.gemm_bf16(A, W, out[0])
     kernels.gemm_bf16(wide[:, :K], W, out[1])
     assert torch.equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("D", [512, 1024, 2048])
+@pytest.mark.parametrize("add", [False, True])
+def test_rmsnorm_rows_equal_those_of_a_large_call(dev, D, add):
+    """One row a workgroup up to 512 rows, one row a wave up to 3072, two above: the same sums per row."""
+    x, d, w = rnd(4099, D, seed=16), rnd(4099, D, seed=17), rnd(D, seed=18)
+    got = []
+    for M in (4099, 3073, 3072, 515, 513, 512, 65, 1):
+        r, out = x[:M].clone(), torch.empty(M, D, dtype=BF, device=dev)
+        kernels.rmsnorm(r, w, 1e-5, out, delta=d[:M] if add else None)
+        got.append((r, out))
+    for r, out in got[1:]:
+        assert torch.equal(out, got[0][1][: len(out)]) and torch.equal(r, got[0][0][: len(r)])

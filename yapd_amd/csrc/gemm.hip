@@ -2011,13 +2011,13 @@ struct NormParams {
   uint16_t* out;
 };
 
-// Two rows per wave; D = 1024 -> 16 bf16 per lane and row (two 16-byte chunks).  All of a
-// wave's loads (both rows and the gain) are requested before the first reduction: one row per
+// kRows rows per wave; D = 1024 -> 16 bf16 per lane and row (two 16-byte chunks).  All of a
+// wave's loads (its rows and the gain) are requested before the first reduction: one row per
 // wave with the gain read after the reduction took 12.1 us at 16384 x 1024 against 11.3 us
-// (four rows per wave: 12.35 us), bit-identical.
+// with two rows (four rows per wave: 12.35 us), bit-identical.
+template <int kRows>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(const NormParams p) {
-  constexpr int kRows = 2;
-  const int row0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * kRows;
+  const int row0 = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * kRows;
   const int lane = threadIdx.x & 63;
   if (row0 >= p.M) return;
   constexpr int kMaxChunks = 4;  // D <= 2048
@@ -2528,7 +2528,17 @@ int rmsnorm_launch(const void* delta, void* residual, const void* x, const void*
                    void* out, hipStream_t st) {
   NormParams p{static_cast<const uint16_t*>(delta), static_cast<uint16_t*>(residual), static_cast<const uint16_t*>(x),
                static_cast<const uint16_t*>(w), eps, M, D, static_cast<uint16_t*>(out)};
-  hipLaunchKernelGGL(rmsnorm_kernel, dim3((M + 7) / 8), dim3(256), 0, st, p);
+  // Few rows: one latency chain per row, on a CU of its own while there are few
+  // (behind the GEMM that wrote x, us, two rows a wave -> this: M = 64 3.26 -> 2.46,
+  // 256 3.73 -> 3.00; four waves of one row each 64 2.76, 600 5.08 -> 4.44, 1000 6.35
+  // -> 5.83, 3000 8.34 -> 7.45, 4096 9.23 -> 9.87).
+  if (M <= 512) {
+    hipLaunchKernelGGL(rmsnorm_kernel<1>, dim3(M), dim3(64), 0, st, p);
+  } else if (M <= 3072) {
+    hipLaunchKernelGGL(rmsnorm_kernel<1>, dim3((M + 3) / 4), dim3(256), 0, st, p);
+  } else {
+    hipLaunchKernelGGL(rmsnorm_kernel<2>, dim3((M + 7) / 8), dim3(256), 0, st, p);
+  }
   YAPD_LAUNCH_CHECK("rmsnorm_kernel launch");
   return YAPD_OK;
 }
