@@ -6,6 +6,7 @@ Bound: bf16 has 8 significant bits, so a rounding moves a value by at most 2^-8 
 P V and the result once more: 2^-8 * sum(p |v|) + 2^-8 * |out| <= 2.1 * 2^-8 * sum(p |v|) with room for the
 fp32 sums (the one-wave kernel reaches 1.65 * 2^-8 on the same inputs)."""
 
+import numpy as np
 import pytest
 import torch
 
@@ -76,3 +77,46 @@ def test_rows_equal_those_of_a_large_call(dev, bl, causal):
         plan.run(q[:n], pool, table[:n], out, 0.125, causal=causal)
         outs.append(out)
     assert torch.equal(outs[0][:5], outs[1])
+
+
+@pytest.mark.parametrize("rows", [2, 97])  # ring and paged kernel
+def test_probabilities_are_summed_in_key_order(dev, rows):
+    """A lane adds its 8 probabilities of a chunk from the first key to the last, the chunk's sum then goes onto the
+    running one: with scores that are whole numbers (q = 1 in one dimension, exp2 of a whole number exact) the sums
+    of every split item follow in fp32, and a sum in another order shows in their last bits."""
+    H, bl = 16, 16
+    lens = [(300, 211)[r % 2] for r in range(rows)]
+    scale = np.float32(0.6931472)  # times log2(e) in fp32: 1
+    for _ in range(4):
+        if scale * np.float32(1.4426950408889634) == 1:
+            break
+        scale = np.nextafter(scale, np.float32(1))
+    assert scale * np.float32(1.4426950408889634) == 1
+    cols = 19
+    rng = np.random.default_rng(rows)
+    score = rng.integers(-24, 1, (rows, H, cols * 16)).astype(np.float32)
+    table = torch.arange(rows * cols, dtype=torch.int32, device=dev).view(rows, cols)
+    pool = torch.zeros(rows * cols, 2, H, 1024, dtype=BF, device=dev)
+    pool[:, 0].view(rows, cols, H, 16, 64)[..., 0] = torch.from_numpy(score).to(dev).view(rows, H, cols, 16).transpose(1, 2).to(BF)
+    q = torch.zeros(rows, bl, H, 64, dtype=BF, device=dev)
+    q[..., 0] = 1
+    plan = AttnPlan(lens, bl, H, torch.device(dev), target_items=4 * rows, min_split_keys=64)
+    plan.run(q, pool, table, torch.empty_like(q), float(scale))
+    work, ml = plan.work.cpu().numpy(), plan.part_ml.cpu().numpy()
+    assert (work[:, 3] >= 0).sum() >= 2 * rows
+    for r, kb, ke, slot in work[work[:, 3] >= 0]:
+        m, l = np.full(H, -np.inf, np.float32), np.zeros((H, 4), np.float32)
+        for k0 in range(kb, ke, 32):
+            s = np.full((H, 32), -np.inf, np.float32)
+            n = min(32, lens[r] - k0)
+            s[:, :n] = score[r, :, k0:k0 + n]
+            mn = np.maximum(m, s.max(1))
+            p = np.exp2(s - mn[:, None]).astype(np.float32).reshape(H, 4, 8)
+            ps = np.zeros((H, 4), np.float32)
+            for i in range(8):
+                ps += p[..., i]
+            l = l * np.exp2(m - mn)[:, None] + ps
+            m = mn
+        want = (l[:, 0] + l[:, 1]) + (l[:, 2] + l[:, 3])
+        assert want.dtype == np.float32
+        assert (ml[slot, :, :, 0] == m).all() and (ml[slot, :, :, 1] == want).all(), (r, kb, ke)

@@ -136,9 +136,13 @@ __device__ __forceinline__ void attn_chunk(const bf16x8_t (&qf)[2], const u32x4_
   const float mref = mn == -INFINITY ? 0.f : mn;
   const float alpha = __builtin_amdgcn_exp2f(m - mref);
   float p[8];
+  float ps = 0.f;  // in key order
 #pragma unroll
-  for (int i = 0; i < 8; ++i) p[i] = __builtin_amdgcn_exp2f(sv[i] - mref);
-  l = l * alpha + (((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7])));
+  for (int i = 0; i < 8; ++i) {
+    p[i] = __builtin_amdgcn_exp2f(sv[i] - mref);
+    ps += p[i];
+  }
+  l = l * alpha + ps;
   m = mn;
   u32x4_t pw;
 #pragma unroll
