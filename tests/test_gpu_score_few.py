@@ -42,3 +42,27 @@ def test_pairs_equal_those_of_a_large_call(dev, bl, cfg, temperature, noise, V):
             ref = res[0][k][:n]
             assert torch.equal(v.nan_to_num(7.5) if v.is_floating_point() else v,
                                ref.nan_to_num(7.5) if ref.is_floating_point() else ref), (n, k)
+
+
+@pytest.mark.parametrize("n", [1, 5, 128])
+@pytest.mark.parametrize("temperature", [0.0, 0.7])
+def test_sampled_tokens_over_the_block(dev, n, temperature):
+    """The sampled tokens may go to the buffer that holds the block: the decision is that of separate buffers."""
+    bl, V = 16, 1001
+    g = torch.Generator(device=dev).manual_seed(n)
+    logits = (torch.randn(n, bl, 1008, generator=g, device=dev) * 3).to(torch.bfloat16)[..., :V]
+    xt = torch.where(torch.rand(n, bl, generator=g, device=dev) > 0.4, V, 7)
+    k_step = torch.full((n,), 2, dtype=torch.int64, device=dev)
+    prior = torch.rand(V, generator=g, device=dev) + 1e-3
+    res = []
+    for over in (False, True):
+        sc = BlockScorer(n_pairs=n, block_size=bl, mask_id=V, stop_id=V - 1, cfg_scale=0.0, time_shift_tau=1.0,
+                         log_prior=BlockScorer.log_prior_from_prior(prior / prior.sum()), device=logits.device)
+        block = xt.clone()
+        if over:
+            sc.out["sampled"] = block
+        r = sc(logits, block, k_step, layout="interleaved", temperature=temperature, seed=11, rng_offset=3)
+        res.append({k: v.clone() for k, v in vars(r).items()})
+    assert res[0]["unmask"].any()
+    for k, v in res[0].items():
+        assert torch.equal(v, res[1][k]), k

@@ -559,9 +559,25 @@ __global__ __launch_bounds__(64) void score_decide_kernel(const ScoreParams P) {
 // 32.5 -> 14.4, 128 40.2 -> 32.9, 192 44.7 -> 45.2; of 16, 5 17.9 -> 11.5, 128
 // 19.9 -> 18.6, 160 21.4 -> 23.0; of 8, 5 12.0 -> 11.3 (without a null row 8.5 ->
 // 9.0), 64 13.0 -> 13.1.
+// The first launch's outputs must not lie over what the second one reads (a
+// caller that samples into the block's own tokens): such calls stay with the one
+// launch, which has a pair's inputs in registers before it writes.
+bool decide_inputs_kept(const ScoreParams& P) {
+  const int64_t items = static_cast<int64_t>(P.n_pairs) * P.bl;
+  const auto apart = [](const void* out, int64_t out_bytes, const void* in, int64_t in_bytes) {
+    const uintptr_t o = reinterpret_cast<uintptr_t>(out), i = reinterpret_cast<uintptr_t>(in);
+    return in == nullptr || o + out_bytes <= i || i + in_bytes <= o;
+  };
+  const auto kept = [&](const void* in, int64_t bytes) {
+    return apart(P.sampled, items * 8, in, bytes) && apart(P.pmi, items * 4, in, bytes);
+  };
+  return kept(P.xt_in, items * 8) && kept(P.k_step, int64_t{P.n_pairs} * 8) && kept(P.active, P.n_pairs) &&
+         kept(P.q_tab, int64_t{P.K} * 4) && kept(P.sched, int64_t{P.K} * 4);
+}
+
 template <bool kHasU, bool kSample, bool kRank = false>
 int launch_score(const ScoreParams& P, hipStream_t st) {
-  if (P.n_pairs <= 128 && P.bl > 8) {
+  if (P.n_pairs <= 128 && P.bl > 8 && decide_inputs_kept(P)) {
     const dim3 grid((P.bl + kItemWaves - 1) / kItemWaves, P.n_pairs);
     hipLaunchKernelGGL((score_item_kernel<kHasU, kSample, kRank>), grid, dim3(64 * kItemWaves), 0, st, P);
     YAPD_LAUNCH_CHECK("score_item_kernel launch");
