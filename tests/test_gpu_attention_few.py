@@ -120,3 +120,31 @@ def test_probabilities_are_summed_in_key_order(dev, rows):
         want = (l[:, 0] + l[:, 1]) + (l[:, 2] + l[:, 3])
         assert want.dtype == np.float32
         assert (ml[slot, :, :, 0] == m).all() and (ml[slot, :, :, 1] == want).all(), (r, kb, ke)
+
+
+@pytest.mark.parametrize("rows", [2, 97])  # ring and paged kernel
+@pytest.mark.parametrize("empty_item", [False, True])
+def test_empty_rows(dev, rows, empty_item):
+    """Device kv_len 0 in the first and last row, with their planned items or with items of no keys: zeros for
+    them, the other rows as without.  The table starts inside a larger buffer, whose other entries are no pages."""
+    H, bl, n = 16, 32, 70
+    g = torch.Generator(device=dev).manual_seed(rows)
+    guard = torch.full((rows + 2, 8), 1 << 30, dtype=torch.int32, device=dev)
+    table = guard[1:-1, :5]
+    table.copy_(torch.randperm(rows * 5, generator=g, device=dev).view(rows, 5))
+    pool = torch.randn(rows * 5, 2, H, 1024, generator=g, device=dev).to(BF)
+    q = torch.randn(rows, bl, H, 64, generator=g, device=dev).to(BF)
+    outs = []
+    for empty in (False, True):
+        plan = AttnPlan([n] * rows, bl, H, torch.device(dev))
+        assert plan.work.shape[0] == rows
+        if empty:
+            plan.kv_len[0] = plan.kv_len[-1] = 0
+            if empty_item:
+                gone = (plan.work[:, 0] == 0) | (plan.work[:, 0] == rows - 1)
+                plan.work[:, 2] = torch.where(gone, plan.work[:, 1], plan.work[:, 2])
+        out = torch.full_like(q, float("nan"))
+        plan.run(q, pool, table, out, 0.125)
+        outs.append(out)
+    assert not outs[1][0].any() and not outs[1][-1].any()
+    assert torch.equal(outs[0][1:-1], outs[1][1:-1])

@@ -221,8 +221,9 @@ struct PageRow {
   int last_page, max_page, lane, base, v;
   __device__ __forceinline__ PageRow(const AttnParams& P, int r, int kvl, int kb, int lane_)
       : tab(P.table + static_cast<int64_t>(r) * P.table_stride),
-        // reads stay inside the row even if kv_len exceeds what the table maps
-        last_page(min((kvl + kPageSize - 1) / kPageSize, P.table_cols) - 1),
+        // reads stay inside the row even if kv_len exceeds what the table maps or is 0 (an empty row's page
+        // is masked or never fetched)
+        last_page(max(min((kvl + kPageSize - 1) / kPageSize, P.table_cols) - 1, 0)),
         max_page(static_cast<int>(min(P.n_pages - 1, int64_t{0x7fffffff}))), lane(lane_) {
     load(min(kb / kPageSize, last_page));
   }
