@@ -40,11 +40,20 @@ def run(dev, rows, bl, H, lens, causal=False, **plan_kw):
 
 
 @pytest.mark.parametrize("bl", [1, 16, 17, 32, 48, 64])
-@pytest.mark.parametrize("rows", [1, 3, 17, 64, 96])  # H = 16: 96 rows are the limit, 64 with bl > 32
+@pytest.mark.parametrize("rows", [1, 3, 17, 64, 96])  # H = 16: 96 rows are the limit, 64 with bl > 32, 24 with bl > 48
 @pytest.mark.parametrize("causal", [False, True])
 def test_few_rows(dev, rows, bl, causal):
     lens = [max(bl, n) for n in ([1, 31, 32, 33, 64, 97, 129, 300, 541] * 11)[:rows]]
     run(dev, rows, bl, 16, lens, causal)
+
+
+@pytest.mark.parametrize("rows", [24, 25, 48, 49])
+@pytest.mark.parametrize("split", [False, True])
+def test_four_tile_limits(dev, rows, split):
+    """Blocks of 64: the ring to 24 rows, to 48 work items above that."""
+    plan = run(dev, rows, 64, 16, [(70, 300, 129)[r % 3] for r in range(rows)],
+               **(dict(target_items=4 * rows, min_split_keys=64) if split else {}))
+    assert (plan.work.shape[0] > 48) == (split or rows > 48)
 
 
 @pytest.mark.parametrize("H", [4, 8, 32])

@@ -395,8 +395,8 @@ attn_ring_kernel(const AttnParams P) {
       const __amdgpu_buffer_rsrc_t r1 = buffer_from(P.pool + kv_plane_offset(page_of(pi + 1), 0, 0, P.H));
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        load_lds16((j & 2) ? r1 : r0, ofs[j < 4 ? j : 4], (j < 4 ? k_plane : v_plane) + (j & 1) * 1024,
-                   ring + st * kStage + j * 1024);
+        load_lds16<true>((j & 2) ? r1 : r0, ofs[j < 4 ? j : 4], (j < 4 ? k_plane : v_plane) + (j & 1) * 1024,
+                         ring + st * kStage + j * 1024);
     };
     for (int c = 0; c < NS && c < n_ch; ++c) issue(c, c);
     if (n_ch > 0) ring_wait<NS - 1>(min(NS - 1, n_ch - 1));
@@ -656,18 +656,27 @@ namespace {
 constexpr int kPagedLds = 64 * 1024;
 
 // The ring kernel while its head-wide workgroups and their waves leave room on
-// the chip (96 rows of 16 heads, 64 with three or four tiles); more rows keep
-// enough page streams in flight with four heads to a workgroup.  Measured (us per
-// launch, paged -> ring; bit-identical): blocks of 32 on 182-632 keys, 2 rows 16.4
-// -> 8.6, 32 23.9 -> 15.5, 96 40.5 -> 34.4, 128 45.1 -> 45.3; causal segments of 64
-// on <= 300 keys, 2 17.3 -> 7.9, 32 19.5 -> 11.2, 64 21.2 -> 19.6, 96 25.7 -> 26.6;
-// blocks of 16 on 64-2048 keys, 8 rows 31.7 -> 17.6, 64 67.2 -> 62.9, 128 114.6 ->
-// 115.5.  By the rows, not the work items, whose count a captured launch does not
-// know.
+// the chip: 96 rows of 16 heads, 64 with three tiles, 24 with four (or, where no
+// more than 48 rows' worth of work items are asked for, three workgroups per CU of
+// their five waves each); more rows keep enough page streams in flight with four
+// heads to a workgroup.  Up to 64 rows it asks for LDS that holds it to four
+// workgroups per CU, as many as unsplit rows need: on long rows six are more
+// scattered page streams at once (64 rows x 16 on 2000-2048 keys 98.8 against 94.6
+// us).  Measured (us per launch, paged -> ring; bit-identical): blocks of 32 on
+// 182-632 keys, 2 rows 18.6 -> 8.0, 32 26.1 -> 13.5, 64 28.1 -> 21.4, 96 39.7 ->
+// 30.4, on 2000-2048 keys 32 51.4 -> 51.1, 64 97.6 -> 97.1, 96 165.9 -> 150.3;
+// blocks of 16 on 64-2048 keys, 64 65.6 -> 56.2, 96 87.2 -> 72.4; causal segments of
+// 64 on <= 300 keys, 2 20.0 -> 7.5, 32 22.2 -> 10.3, 48 22.5 -> 15.1, blocks of 64 on
+// 2000-2048 keys, 24 62.5 -> 49.2, 28 56.4 -> 62.5 (not taken).  The kernel reads K/V
+// with non-temporal loads as the paged one does: without, 64 rows x 32 on 2000-2048
+// keys take 115 us and 32 rows 56.  A captured launch gives the capacity of its work
+// list for n_work, the same on every replay.
 template <int NQT>
 void launch_paged(const AttnParams& P, int n_work, hipStream_t st) {
-  if (static_cast<int64_t>(P.rows) * P.H <= (NQT >= 3 ? 1024 : 1536) && n_work <= INT32_MAX / P.H) {
-    hipLaunchKernelGGL(attn_ring_kernel<NQT>, dim3(n_work * P.H), dim3(64 * (NQT + 1)), kRing * kRingStage, st, P);
+  const int64_t row_heads = static_cast<int64_t>(P.rows) * P.H, wgs = static_cast<int64_t>(n_work) * P.H;
+  if ((row_heads <= (NQT == 4 ? 384 : NQT == 3 ? 1024 : 1536) || (NQT == 4 && wgs <= 768)) && wgs <= INT32_MAX) {
+    const int lds = row_heads <= 1024 ? 40 * 1024 : kRing * kRingStage;
+    hipLaunchKernelGGL(attn_ring_kernel<NQT>, dim3(n_work * P.H), dim3(64 * (NQT + 1)), lds, st, P);
   } else {
     hipLaunchKernelGGL(attn_paged_kernel<NQT>, dim3(n_work * (P.H / kWaves)), dim3(64 * kWaves), kPagedLds, st, P);
   }

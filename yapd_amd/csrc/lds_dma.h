@@ -19,11 +19,12 @@ __device__ __forceinline__ void load_lds16(const uint16_t* src, char* lds_run) {
 // (ofs per lane, sofs uniform).  A buffer load is no FLAT instruction, so the
 // compiler's waits for LDS reads stay counted ones; with global_load_lds in
 // flight it waits for every LDS read outstanding (lgkmcnt(0)) before each use
-// of a fragment.
+// of a fragment.  kStream: a non-temporal load, for bytes read once.
+template <bool kStream = false>
 __device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t rsrc, uint32_t ofs, uint32_t sofs, char* lds_run) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(
       rsrc, reinterpret_cast<__attribute__((address_space(3))) void*>(reinterpret_cast<uintptr_t>(lds_run)), 16, ofs,
-      sofs, 0, 0);
+      sofs, 0, kStream ? 2 : 0);
 }
 
 // Descriptor over the 4 GiB from p on (word 3: raw 32-bit elements, no swizzle).
