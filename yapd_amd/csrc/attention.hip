@@ -650,11 +650,6 @@ extern "C" int yapd_attn_plan(const int32_t* kv_len, int rows, int target_items,
 namespace yapd {
 namespace {
 
-// LDS asked for only to hold attn_paged_kernel to two workgroups per CU: three
-// (one-tile blocks would fit them) are more scattered page streams at once, 256
-// rows x 16 on 116-317 keys 45.1 against 43.4 us, x 8 on 100-600 53.5 against 51.9.
-constexpr int kPagedLds = 64 * 1024;
-
 // The ring kernel while its head-wide workgroups and their waves leave room on
 // the chip: 96 rows of 16 heads, 64 with three tiles, 24 with four (or, where no
 // more than 48 rows' worth of work items are asked for, three workgroups per CU of
@@ -678,7 +673,7 @@ void launch_paged(const AttnParams& P, int n_work, hipStream_t st) {
     const int lds = row_heads <= 1024 ? 40 * 1024 : kRing * kRingStage;
     hipLaunchKernelGGL(attn_ring_kernel<NQT>, dim3(n_work * P.H), dim3(64 * (NQT + 1)), lds, st, P);
   } else {
-    hipLaunchKernelGGL(attn_paged_kernel<NQT>, dim3(n_work * (P.H / kWaves)), dim3(64 * kWaves), kPagedLds, st, P);
+    hipLaunchKernelGGL(attn_paged_kernel<NQT>, dim3(n_work * (P.H / kWaves)), dim3(64 * kWaves), 0, st, P);
   }
 }
 
