@@ -33,11 +33,11 @@ def test_pairs_equal_those_of_a_large_call(dev, bl, cfg, temperature, noise, V):
     sc = BlockScorer(n_pairs=BIG, block_size=bl, mask_id=V, stop_id=V - 1, cfg_scale=cfg, time_shift_tau=1.0,
                      log_prior=BlockScorer.log_prior_from_prior(prior / prior.sum()), device=logits.device)
     res = []
-    for n in (BIG, 128, 5, 1):
+    for n in (BIG, 128, 65, 64, 5, 1):
         r = sc(logits[: n * rows // BIG, :, :V], xt[:n], k_step[:n], layout="interleaved", active=active[:n],
                temperature=temperature, position_noise=noise, seed=11, rng_offset=3, n_pairs=n)
         res.append({k: v.clone() for k, v in vars(r).items()})
-    for n, r in zip((128, 5, 1), res[1:]):
+    for n, r in zip((128, 65, 64, 5, 1), res[1:]):
         for k, v in r.items():
             ref = res[0][k][:n]
             assert torch.equal(v.nan_to_num(7.5) if v.is_floating_point() else v,

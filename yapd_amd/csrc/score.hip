@@ -558,7 +558,12 @@ __global__ __launch_bounds__(64) void score_decide_kernel(const ScoreParams P) {
 // null row, pair kernel -> two launches): blocks of 32, 1 pair 30.7 -> 11.1, 32
 // 32.5 -> 14.4, 128 40.2 -> 32.9, 192 44.7 -> 45.2; of 16, 5 17.9 -> 11.5, 128
 // 19.9 -> 18.6, 160 21.4 -> 23.0; of 8, 5 12.0 -> 11.3 (without a null row 8.5 ->
-// 9.0), 64 13.0 -> 13.1.
+// 9.0), 64 13.0 -> 13.1.  The least work a position can be, the argmax of one row,
+// pays for the second launch only to 64 pairs in blocks of up to 12: of 9, 64 9.3 ->
+// 9.2, 96 9.6 -> 10.4; of 12, 64 9.7 -> 9.7, 128 10.3 -> 11.2; of 13 and more, 128
+// 11.9 -> 11.8.  Sampling is the most: blocks of 16, 128 pairs 67 -> 41.  Those are
+// at 8194 tokens; at 1001 the argmax over blocks of up to 16 is not worth a second
+// launch (of 12, 1 pair 6.3 -> 7.1, of 16, 32 7.4 -> 7.7).
 // The first launch's outputs must not lie over what the second one reads (a
 // caller that samples into the block's own tokens): such calls stay with the one
 // launch, which has a pair's inputs in registers before it writes.
@@ -577,7 +582,9 @@ bool decide_inputs_kept(const ScoreParams& P) {
 
 template <bool kHasU, bool kSample, bool kRank = false>
 int launch_score(const ScoreParams& P, hipStream_t st) {
-  if (P.n_pairs <= 128 && P.bl > 8 && decide_inputs_kept(P)) {
+  const bool least = !kSample && P.bl <= 16 && P.vocab < 8192;
+  const int max_pairs = least ? 0 : !kHasU && !kSample && P.bl <= 12 ? 64 : 128;
+  if (P.n_pairs <= max_pairs && P.bl > 8 && decide_inputs_kept(P)) {
     const dim3 grid((P.bl + kItemWaves - 1) / kItemWaves, P.n_pairs);
     hipLaunchKernelGGL((score_item_kernel<kHasU, kSample, kRank>), grid, dim3(64 * kItemWaves), 0, st, P);
     YAPD_LAUNCH_CHECK("score_item_kernel launch");
