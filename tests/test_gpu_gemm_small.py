@@ -92,6 +92,40 @@ def test_short_and_odd_k(dev, K, M):
     assert ((C.double() - ref).abs() <= ref.abs() * 2.0 ** -8 + mag * K * 2.0 ** -24).all()
 
 
+@pytest.mark.parametrize("K", [64, 128, 192, 320, 512, 576, 1088, 1344, 2048])
+def test_short_k_rows_equal_the_large_tiles(dev, K):
+    """129 to 256 tiles of 128 x 128: three stages of gemm_dl_kernel at short K, gemm_sk_kernel above, whose limit
+    depends on the epilogue; one k-tile, as many as the stages hold, and more."""
+    A, W, R = rnd(BIG, K, std=0.5, seed=19), rnd(1024, K, std=0.02, seed=20), rnd(BIG, 1024, seed=21)
+    for f in (kernels.gemm_bf16, kernels.gemm_bf16_residual):
+        got = [R[:M].clone() for M in (BIG, 3001)]
+        for C in got:
+            f(A[: len(C)], W, C)
+        assert torch.equal(got[0][:3001], got[1]), f.__name__
+    W = rnd(8192, K, std=0.02, seed=22)
+    act = [torch.empty(M, 4096, dtype=BF, device=dev) for M in (8192, 461)]
+    for o in act:
+        kernels.gemm_swiglu(A[: len(o)], W, o)
+    assert torch.equal(act[0][:461], act[1])
+
+
+@pytest.mark.parametrize("D", [64, 512, 1088])
+def test_short_k_qkv_rows_equal_the_large_tiles(dev, D):
+    H, bl, big, rows = 8, 32, 1024, 60
+    A, W = rnd(big * bl, D, seed=23), rnd(3 * H * 64, D, std=0.02, seed=24)
+    fr = torch.outer(torch.arange(400.0), 10000.0 ** (-torch.arange(0, 64, 2) / 64))
+    cos, sin = (torch.cat([f, f], -1).to(BF).float().to(dev) for f in (fr.cos(), fr.sin()))
+    pos0 = torch.arange(big, dtype=torch.int32, device=dev) % 77
+    table = torch.arange(big * 8, dtype=torch.int32, device=dev).view(big, 8)
+    got = []
+    for n in (big, rows):
+        pool = torch.zeros(big * 8, 2, H, 1024, dtype=BF, device=dev)
+        q = torch.empty(n * bl, H * 64, dtype=BF, device=dev)
+        kernels.gemm_qkv_rope_kv(A[: n * bl], W, cos, sin, pos0[:n], bl, q, pool, table[:n])
+        got.append((q[: rows * bl], pool[: rows * 8]))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 def test_wide_row_pitch(dev):
     """Rows further apart than 32-bit offsets in a tile reach: the same values as a packed call."""
     M, N, K = 5, 64, 128

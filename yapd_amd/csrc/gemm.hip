@@ -669,7 +669,7 @@ __global__ __launch_bounds__(T::THREADS) void gemm_kernel(const GemmParams p) {
 // bank groups (two 128-byte rows share one 256-byte bank line).  A load
 // instruction covers 8 rows; lane i writes slot i % 8 of row i / 8, so it
 // fetches the chunk that belongs there.
-template <class T>
+template <class T, int NS = 2>
 struct DlLayout {
   static_assert(T::BK == 64, "direct-load tiles use 128-byte LDS rows");
   static constexpr int WAVES = T::THREADS / 64;
@@ -682,20 +682,23 @@ struct DlLayout {
   static constexpr int LA = T::BM / 8 / WAVES;  // 1 KB loads per wave and k-tile
   static constexpr int LB = T::BN / 8 / WAVES;
   static_assert(LA * 8 * WAVES == T::BM && LB * 8 * WAVES == T::BN, "rows must split evenly over the waves");
+  static constexpr int LPT = LA + LB;
+  static_assert((NS == 2 || NS == 3) && LPT <= 63, "two or three stages; the vmcnt counter holds at most 63 loads");
   static constexpr int C_BYTES = T::BM * (T::BN + 8) * 2;  // store-epilogue staging
-  static constexpr int LDS = 2 * STAGE > C_BYTES ? 2 * STAGE : C_BYTES;
+  static constexpr int LDS = NS * STAGE > C_BYTES ? NS * STAGE : C_BYTES;
 };
 
-// Hand-off of an LDS stage across the workgroup: this wave's loads have landed
-// and its LDS reads have completed (so the stage it read last may be
-// overwritten), then the workgroup barrier.
+// Hand-off of an LDS stage across the workgroup: at most N of this wave's loads,
+// later tiles', are in flight and its LDS reads have completed (so the stage it
+// read last may be overwritten), then the workgroup barrier.
+template <int N>
 __device__ __forceinline__ void stage_barrier() {
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-template <class T, int EPI, int AM>
+template <class T, int EPI, int AM, int NS>
 __global__ __launch_bounds__(T::THREADS) void gemm_dl_kernel(const GemmParams p) {
-  using L = DlLayout<T>;
+  using L = DlLayout<T, NS>;
   // Dynamic LDS: the compiler cannot see the DMA writes into a static
   // __shared__ array and would treat its contents as undefined.
   extern __shared__ __attribute__((aligned(16))) uint16_t dyn_lds[];
@@ -809,18 +812,28 @@ __global__ __launch_bounds__(T::THREADS) void gemm_dl_kernel(const GemmParams p)
     __builtin_amdgcn_sched_group_barrier(0x008, T::TM * T::TN - (T::TM + T::TN), 0);
   };
 
-  // Two LDS stages: tile kt + 1 is requested at the top of tile kt into the stage
-  // tile kt - 1 used (its last fragments were consumed by the MFMAs that ended
-  // it); the barrier before its first fragments are read waits for its loads.
+  // NS LDS stages: tile kt + NS - 1 is requested at the top of tile kt into the stage
+  // tile kt - 1 used (its last fragments were consumed by the MFMAs that ended it);
+  // the barrier before the first fragments of tile kt + 1 are read waits for its
+  // loads and leaves those of tile kt + 2 (three stages) in flight.
   const int kt_n = p.K / T::BK;
   issue(0, 0);
+  if (NS == 3 && kt_n > 1) issue(1, 1);
   const RowMeta rm = EPI == kEpiQkv ? qkv_row_meta<T>(p, m0, tid) : RowMeta{0, 0};
-  stage_barrier();
+  const auto hand_over = [&](bool later) {  // uniform: every wave takes the same barrier
+    if (NS == 3 && later) {
+      stage_barrier<L::LPT>();
+    } else {
+      stage_barrier<0>();
+    }
+  };
+  hand_over(kt_n > 1);
   read_frags(0, 0, 0);
+  int stage = 0;
   for (int kt = 0; kt < kt_n; ++kt) {
-    const int stage = kt & 1;
     const bool more = kt + 1 < kt_n;
-    if (more) issue(kt + 1, stage ^ 1);
+    const int next = stage + 1 == NS ? 0 : stage + 1;
+    if (kt + NS - 1 < kt_n) issue(kt + NS - 1, stage == 0 ? NS - 1 : stage - 1);
 #pragma unroll
     for (int ks = 0; ks + 1 < KS; ++ks) {
       read_frags(stage, ks + 1, (ks + 1) & 1);
@@ -828,10 +841,11 @@ __global__ __launch_bounds__(T::THREADS) void gemm_dl_kernel(const GemmParams p)
       interleave();
     }
     // after the last tile: every wave is done with the stages before the epilogue reuses LDS
-    stage_barrier();
-    if (more) read_frags(stage ^ 1, 0, 0);
+    hand_over(kt + 2 < kt_n);
+    if (more) read_frags(next, 0, 0);
     mfma_step((KS - 1) & 1);
     if (more) interleave();
+    stage = next;
   }
   static_assert(EPI != kEpiQkv || qkv_lds_bytes<T>() <= L::LDS, "qkv epilogue LDS");
   finish_tile<T, EPI>(p, acc, dyn_lds, rm, m0, n0, wm, wn, lane, tid);
@@ -2105,23 +2119,23 @@ int launch_tile(const GemmParams& p, hipStream_t st) {
   return YAPD_OK;
 }
 
-template <class T, int EPI, int AM>
+template <class T, int EPI, int AM, int NS = 2>
 int launch_dl(const GemmParams& p, hipStream_t st) {
-  using L = DlLayout<T>;
+  using L = DlLayout<T, NS>;
   // The dynamic-LDS limit is raised once per kernel and device (setting it
   // twice, e.g. from two threads, is harmless).
   static bool lds_set[64] = {false};
   int dev = 0;
   if (int rc = check_hip(hipGetDevice(&dev), "hipGetDevice")) return rc;
   if (dev < 0 || dev >= 64 || !lds_set[dev]) {
-    if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dl_kernel<T, EPI, AM>),
+    if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dl_kernel<T, EPI, AM, NS>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, L::LDS),
                            "gemm_dl_kernel LDS attribute"))
       return rc;
     if (dev >= 0 && dev < 64) lds_set[dev] = true;
   }
   const dim3 grid((p.N + T::BN - 1) / T::BN, (p.M + T::BM - 1) / T::BM), block(T::THREADS);
-  hipLaunchKernelGGL((gemm_dl_kernel<T, EPI, AM>), grid, block, L::LDS, st, p);
+  hipLaunchKernelGGL((gemm_dl_kernel<T, EPI, AM, NS>), grid, block, L::LDS, st, p);
   YAPD_LAUNCH_CHECK("gemm_dl_kernel launch");
   return YAPD_OK;
 }
@@ -2347,16 +2361,25 @@ int launch_gemm(GemmParams p, hipStream_t st) {
     if (sk_fits<Sk64x32>(p, cus)) return launch_sk<Sk64x32, EPI, AM>(p, st);
     if (sk_fits<Sk64>(p, cus)) return launch_sk<Sk64, EPI, AM>(p, st);
     if (sk_fits<Sk128x64>(p, cus)) return launch_sk<Sk128x64, EPI, AM>(p, st);
-    if (sk_fits<Sk128>(p, cus)) return launch_sk<Sk128, EPI, AM>(p, st);
-  }
-  // In between, 128 x 128 tiles of 8 waves, two workgroups of two stages per CU
-  // (down 61 us against 83 us with three stages at M = 6144); the quantised path
-  // keeps the register-staged kernel, which dequantises W on its way into LDS.
-  const int64_t small_tiles = static_cast<int64_t>((p.M + 127) / 128) * ((p.N + 127) / 128);
-  p.xcd_band = small_tiles <= cus ? 1 : 0;
-  if constexpr (BQ == 0) {
+    if (sk_fits<Sk128>(p, cus)) {
+      // The 128 x 128 tile's k-step is the faster one, but from registers its 32 KB of
+      // C take longer than from LDS: below these K gemm_dl_kernel's tile of three
+      // stages is ahead (us, it -> gemm_sk_kernel: residual N = 1024, M = 3000, K = 64
+      // 5.8 -> 8.5, 1024 14.1 -> 15.4, 1344 17.3 -> 17.6, 2048 22.6 -> 21.7; store K =
+      // 320 7.9 -> 8.5, 1024 13.6 -> 12.8; SwiGLU K = 64 4.8 -> 5.3, 1024 13.0 -> 11.9;
+      // QKV of 8 heads, M = 2048, K = 512 11.9 -> 13.3, of 16, M = 1280, K = 1088 17.5
+      // -> 17.9, of 32, M = 640, K = 2048 26.8 -> 25.0).
+      constexpr int kMinK = EPI == kEpiResidual ? 2048 : EPI == kEpiQkv ? 1536 : EPI == kEpiStore ? 576 : 512;
+      if (p.K >= kMinK) return launch_sk<Sk128, EPI, AM>(p, st);
+      p.xcd_band = 1;
+      return launch_dl<TileM, EPI, AM, 3>(p, st);
+    }
+    // In between, 128 x 128 tiles of 8 waves, two workgroups of two stages per CU
+    // (down 61 us against 83 us with three stages at M = 6144).
+    p.xcd_band = 0;
     return launch_dl<TileM, EPI, AM>(p, st);
   } else {
+    const int64_t small_tiles = static_cast<int64_t>((p.M + 127) / 128) * ((p.N + 127) / 128);
     // Quantised W: the same rule on gemm_skq_kernel's tiles.  Measured (us, one
     // graph of 24 calls over 12 weights, 4 bits; 128 x 128 tiles of
     // gemm_dlq_kernel before -> now, bit-identical): QKV M = 64 12.9 -> 5.9, 400
