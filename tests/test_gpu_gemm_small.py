@@ -150,3 +150,16 @@ def test_rmsnorm_rows_equal_those_of_a_large_call(dev, D, add):
         got.append((r, out))
     for r, out in got[1:]:
         assert torch.equal(out, got[0][1][: len(out)]) and torch.equal(r, got[0][0][: len(r)])
+
+
+@pytest.mark.parametrize("N", [1, 2, 63, 64, 65, 255, 257])
+def test_few_columns_of_many_rows(dev, N):
+    """One 256 x 256 tile per CU and no more columns than a last column tile that is split off holds: the bound of
+    test_short_and_odd_k."""
+    M, K = 65536, 128
+    A, W = rnd(M, K, seed=25), rnd(N, K, std=0.1, seed=26)
+    C = torch.full((M, N), float("nan"), dtype=BF, device=dev)
+    kernels.gemm_bf16(A, W, C)
+    ref = A.double() @ W.double().T
+    mag = A.double().abs() @ W.double().abs().T
+    assert ((C.double() - ref).abs() <= ref.abs() * 2.0 ** -8 + mag * K * 2.0 ** -24).all()

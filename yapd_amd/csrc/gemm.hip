@@ -2290,7 +2290,7 @@ int launch_gemm(GemmParams p, hipStream_t st) {
       if constexpr (EPI == kEpiStore) {
         // the head's last 2 columns (N = 8194) as below: their own launch
         const int tail = p.N % 256;
-        if (tail != 0 && tail <= 64) {
+        if (p.N > 64 && tail != 0 && tail <= 64) {
           GemmParams rest = p;
           p.N -= tail;
           rest.W = p.W + static_cast<int64_t>(p.N) * p.ldw;
