@@ -43,3 +43,20 @@ def test_strided_rows(dev, bits):
     qgemm_affine(wide[:, :1024], *codes, bits, out=out[:, :200])
     assert torch.equal(out[:, :200], qgemm_affine(A, *codes, bits))
     assert (out[:, 200:] == 7.0).all()
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("N,K", [(1024, 64), (1000, 128), (3072, 192), (200, 704), (1024, 832), (1024, 896), (1024, 1088),
+                                 (1024, 1152), (136, 9216), (520, 16384)])
+def test_k_outside_the_rings(dev, bits, N, K):
+    """K too short for the ring, and too long for its scales: 128 x 128 tiles of gemm_dlq_kernel, of which one k-tile
+    is the shortest.  Against fp64 on the dequantised weights, half a bf16 ulp and the error of K fp32 sums, and bit
+    for bit between row counts."""
+    A, codes = inputs(dev, 4000, N, K, bits)
+    W = dequant_affine(*codes, bits).double()
+    got = [qgemm_affine(A[:M], *codes, bits) for M in (4000, 1000, 129, 3)]
+    for C in got[1:]:
+        assert torch.equal(C, got[0][: len(C)]), len(C)
+    A = A[:1000].double()
+    ref, mag = A @ W.T, A.abs() @ W.abs().T
+    assert ((got[1].double() - ref).abs() <= ref.abs() * 2.0 ** -8 + mag * K * 2.0 ** -24).all()

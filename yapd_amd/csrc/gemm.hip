@@ -7,14 +7,16 @@
 //   * gemm_pt_kernel: 256 x 256 tiles, one persistent 4-wave workgroup per CU
 //     (at least two tiles per CU, one with the plain or residual epilogue);
 //   * gemm_dl_kernel: 256 x 256 tiles of 8 waves that fill three quarters of the
-//     CUs, and 128 x 128 tiles where those give more than one per CU;
+//     CUs, and 128 x 128 tiles where those give more than one per CU, or at most
+//     one at short K;
 //   * gemm_sk_kernel: 16 x 16 to 128 x 128 tiles, the smallest with at most one
 //     workgroup per CU, as many LDS stages as fit (small and mid M).
 // A and W k-slices go global -> LDS by direct loads.  Affine-quantised W:
 // gemm_dlq_kernel (256 x 256 tiles that fill the CUs, W dequantised from registers
-// into LDS), gemm_skq_kernel (up to one workgroup per CU: gemm_sk_kernel's tiles,
-// W dequantised from LDS into LDS) and, between them, gemm_kernel (register-staged
-// 128 x 128 tiles with padded LDS rows).  Every kernel sums K in the same order, so a row's
+// into LDS; 128 x 128 ones, up to one per CU, at K that the next does not take),
+// gemm_skq_kernel (up to one workgroup per CU: gemm_sk_kernel's tiles, W dequantised
+// from LDS into LDS) and, between them, gemm_kernel (register-staged 128 x 128 tiles
+// with padded LDS rows).  Every kernel sums K in the same order, so a row's
 // result does not depend on which kernel the batch size selects.  K advances in
 // steps of 64.
 //
@@ -1485,8 +1487,9 @@ __global__ __launch_bounds__(Q::T::THREADS) void gemm_skq_kernel(const GemmParam
 }
 
 // Affine-quantised W on the direct-load layout: A moves global -> LDS by
-// direct loads as in gemm_dl_kernel; W's codes (16-byte chunks), scales and biases
-// come into registers one k-tile ahead, and after the k-tile's MFMAs each thread dequantises its
+// direct loads as in gemm_dl_kernel; W's codes (16-byte chunks, 8-byte ones where
+// 16-byte ones would not give every thread one: 4-bit codes on 128-column tiles),
+// scales and biases come into registers one k-tile ahead, and after the k-tile's MFMAs each thread dequantises its
 // chunk (w = scale * q + bias, rounded once to bf16, as in gemm_kernel) and
 // writes it into the next stage's B tile in the same swizzled layout, so the
 // fragment reads and the MFMA loop are gemm_dl_kernel's.  Only W passes
@@ -1518,10 +1521,11 @@ __global__ __launch_bounds__(T::THREADS) void gemm_dlq_kernel(const GemmParams p
     for (int j = 0; j < L::LA; ++j) load_lds16(a_src[j] + kt * T::BK, a_dst + j * 1024);
   };
 
-  // W codes: a 16-byte chunk holds QVALS codes of one row; a row's k-tile (one
-  // quantisation group of 64) is QCH chunks; each thread owns CQ chunks.
-  constexpr int QW = 4;  // 32-bit words per chunk
-  constexpr int QVALS = 128 / BQ;
+  // W codes: a chunk of QB bytes holds QVALS codes of one row; a row's k-tile
+  // (one quantisation group of 64) is QCH chunks; each thread owns CQ chunks.
+  constexpr int QB = (T::BN * (T::BK * BQ / 128)) % T::THREADS == 0 ? 16 : 8;
+  constexpr int QW = QB / 4;  // 32-bit words per chunk
+  constexpr int QVALS = QB * 8 / BQ;
   constexpr int QCH = T::BK / QVALS;
   constexpr int CQ = T::BN * QCH / T::THREADS;
   static_assert(CQ >= 1 && CQ * T::THREADS == T::BN * QCH, "quantised tile loads must divide evenly");
@@ -1546,9 +1550,15 @@ __global__ __launch_bounds__(T::THREADS) void gemm_dlq_kernel(const GemmParams p
 #pragma unroll
     for (int c = 0; c < CQ; ++c) {
       const uint32_t* src = q_src[c] + kt * T::BK * BQ / 32;
-      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(src);
+      if constexpr (QW == 4) {
+        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(src);
 #pragma unroll
-      for (int w = 0; w < QW; ++w) rq[c][w] = v[w];
+        for (int w = 0; w < 4; ++w) rq[c][w] = v[w];
+      } else {
+        const u32x2_t v = *reinterpret_cast<const u32x2_t*>(src);
+        rq[c][0] = v[0];
+        rq[c][1] = v[1];
+      }
       rs[c] = s_src[c][kt];
       rz[c] = z_src[c][kt];
     }
@@ -2398,10 +2408,20 @@ int launch_gemm(GemmParams p, hipStream_t st) {
     if (skq_fits<Skq64x32<BQ>>(p, cus)) return launch_skq<Skq64x32<BQ>, EPI, BQ>(p, st);
     if (skq_fits<Skq64<BQ>>(p, cus)) return launch_skq<Skq64<BQ>, EPI, BQ>(p, st);
     if (skq_fits<Skq128x64<BQ>>(p, cus)) return launch_skq<Skq128x64<BQ>, EPI, BQ>(p, st);
-    if (skq_fits<Skq128<BQ>>(p, cus)) return launch_skq<Skq128<BQ>, EPI, BQ>(p, st);
-    // Larger grids (o at M = 8192: 29.3 us against 32.5 with gemm_dlq_kernel's
-    // 128 x 128 tiles) and K of fewer k-tiles than the rings hold.
-    p.xcd_band = small_tiles <= cus ? 1 : 0;
+    if ((p.K >= 1152 || (p.K >= 896 && 2 * small_tiles > cus)) && skq_fits<Skq128<BQ>>(p, cus))
+      return launch_skq<Skq128<BQ>, EPI, BQ>(p, st);
+    // What is left of at most one 128 x 128 tile per CU runs on gemm_dlq_kernel: K so
+    // short that the ring's prologue shows (us, it -> gemm_skq_kernel, N = 3072, 4 bits:
+    // K = 192, M = 16 5.0 -> 5.4, 512 5.8 -> 7.7; K = 704, M = 512 11 % slower, K =
+    // 1088 4 %; with most CUs at work the 128 x 128 ring is ahead from K = 896 on: M =
+    // 1000 7 % faster, at K = 640 the same) and K whose scales do not fit beside the
+    // ring (N = 1024, 8 bits, K = 8768, M = 64 123 us, gemm_kernel 139; M = 3000 135,
+    // 162).  Larger grids: gemm_kernel (o at M = 8192: 29.3 us against 32.5).
+    if (small_tiles <= cus) {
+      p.xcd_band = 1;
+      return launch_dlq<TileM, EPI, AM, BQ>(p, st);
+    }
+    p.xcd_band = 0;
     return launch_tile<TileS, EPI, AM, BQ>(p, st);
   }
 }
