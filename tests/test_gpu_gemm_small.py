@@ -19,9 +19,9 @@ def rnd(*shape, std=1.0, seed=0):
     return (torch.randn(*shape, generator=g, device="cuda") * std).to(BF)
 
 
-# N = 1024: 16 x 16 up to M = 128, 32 x 32 to 256, 64 x 32 to 512, 64 x 64 to 1024, 128 x 64 to 2048,
-# 128 x 128 to 4096
-SIZES = (1, 15, 17, 64, 128, 129, 256, 257, 511, 513, 1000, 1025, 1900, 2049, 3000, 4096)
+# N = 1024: 16 x 16 up to M = 64, 32 x 16 to 128, 32 x 32 to 256, 64 x 32 to 512, 64 x 64 to 1024, 128 x 64 to
+# 2048, 128 x 128 to 4096
+SIZES = (1, 15, 17, 64, 65, 100, 113, 127, 128, 129, 256, 257, 511, 513, 1000, 1025, 1900, 2049, 3000, 4096)
 
 
 @pytest.mark.parametrize("epi", ["store", "residual"])
@@ -126,16 +126,35 @@ def test_short_k_qkv_rows_equal_the_large_tiles(dev, D):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
-def test_wide_row_pitch(dev):
-    """Rows further apart than 32-bit offsets in a tile reach: the same values as a packed call."""
-    M, N, K = 5, 64, 128
-    wide = torch.empty(M, (1 << 22) + 8, dtype=BF, device=dev)
+@pytest.mark.parametrize("epi,which", [("store", "A"), ("store", "W"), ("residual", "A"), ("residual", "W"),
+                                       ("swiglu", "A"), ("qkv", "A"), ("head", "W")])  # others take packed rows only
+def test_wide_row_pitch(dev, epi, which):
+    """Rows of A or W further apart than 32-bit offsets in a tile reach: the same values as a packed call."""
+    H, rows, bl, K = 4, 3, 43, 128  # 129 rows: two row tiles, the second of one row
+    M, N = rows * bl, {"qkv": 3 * H * 64}.get(epi, 256)
     A, W = rnd(M, K, seed=14), rnd(N, K, std=0.02, seed=15)
-    wide[:, :K] = A
-    out = [torch.empty(M, N, dtype=BF, device=dev) for _ in range(2)]
-    kernels.gemm_bf16(A, W, out[0])
-    kernels.gemm_bf16(wide[:, :K], W, out[1])
-    assert torch.equal(out[0], out[1])
+    n_wide = M if which == "A" else N
+    wide = torch.empty(n_wide, (1 << 22) + 8, dtype=BF, device=dev)[:, :K]
+    wide.copy_(A if which == "A" else W)
+    table = torch.arange(rows * 4, dtype=torch.int32, device=dev).view(rows, 4)
+    pos0 = torch.tensor([0, 5, 16], dtype=torch.int32, device=dev)
+    cos, sin = rnd(64, 64, seed=27).float(), rnd(64, 64, seed=28).float()
+    got = []
+    for a, w in ((A, W), (wide, W) if which == "A" else (A, wide)):
+        if epi == "qkv":
+            C, pool = torch.empty(M, H * 64, dtype=BF, device=dev), torch.zeros(rows * 4, 2, H, 1024, dtype=BF, device=dev)
+            kernels.gemm_qkv_rope_kv(a, w, cos, sin, pos0, bl, C, pool, table)
+            got.append((C, pool))
+        elif epi == "head":
+            C = torch.empty(rows, bl, N, dtype=BF, device=dev)
+            kernels.gemm_head_shift(a.view(rows, bl, K), rnd(rows, 1, K, seed=29), w, C)
+            got.append((C,))
+        else:
+            C = rnd(M, N // 2 if epi == "swiglu" else N, seed=30)
+            {"store": kernels.gemm_bf16, "residual": kernels.gemm_bf16_residual, "swiglu": kernels.gemm_swiglu}[epi](a, w, C)
+            got.append((C,))
+    for x, y in zip(*got):
+        assert torch.equal(x, y)
 
 
 @pytest.mark.parametrize("D", [512, 1024, 2048])

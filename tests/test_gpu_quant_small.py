@@ -21,15 +21,16 @@ def inputs(dev, M, N, K, bits):
 
 
 @pytest.mark.parametrize("bits", [4, 8])
-# 1024: 16 x 16 tiles up to M = 128, 32 x 32 to 256, 64 x 32 to 512, 64 x 64 to 1024, 128 x 64 to 2048, 128 x 128 to
-# 4096.  K: one stage short of the deep tiles' rings (768, 192), odd numbers of k-tiles, scales past one batch (4096)
-@pytest.mark.parametrize("N,K", [(1024, 1024), (1000, 4096), (72, 768), (1024, 192), (200, 1344), (3072, 512)])
+# N = 1024: 16 x 16 tiles up to M = 64, 32 x 16 to 128, 32 x 32 to 256, 64 x 32 to 512, 64 x 64 to 1024, 128 x 64 to
+# 2048 (not at 8 bits and K = 4096, whose scales do not fit beside its ring), 128 x 128 to 4096.  K: one stage short
+# of the deep tiles' rings (768, 192), odd numbers of k-tiles, scales past one batch (4096)
+@pytest.mark.parametrize("N,K", [(1024, 1024), (1000, 4096), (1024, 2048), (72, 768), (1024, 192), (200, 1344), (3072, 512)])
 def test_rows_equal_the_bf16_gemm_on_dequantised_weights(dev, bits, N, K):
     A, codes = inputs(dev, 4096, N, K, bits)
     W = dequant_affine(*codes, bits)
     ref = torch.empty(4096, N, dtype=BF, device=dev)
     kernels.gemm_bf16(A, W, ref)
-    for M in (1, 15, 16, 17, 64, 128, 129, 256, 257, 511, 513, 1000, 1025, 1900, 2049, 3000, 4096):
+    for M in (1, 15, 16, 17, 64, 65, 100, 113, 127, 128, 129, 256, 257, 511, 513, 1000, 1025, 1900, 2049, 3000, 4096):
         assert torch.equal(qgemm_affine(A[:M], *codes, bits), ref[:M]), M
 
 

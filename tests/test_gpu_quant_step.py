@@ -27,6 +27,7 @@ import torch
 
 from oracle import llama as OL
 from test_gpu_step import BL, PAIRS, ROWS, decisions_vs_oracle
+from yapd_amd import kernels
 from yapd_amd.engines.hip import HipEngine
 from yapd_amd.quant import quantize_affine
 from yapd_amd.step import DecodeStep
@@ -90,8 +91,8 @@ def replay(w):
 # 16384 tokens) the engine dequantises each layer's weights once into its
 # scratch and runs the bf16 kernels; with fused=True (no scratch) and at 16
 # pairs (1024 rows) the fused kernels run: at 256 pairs every projection on
-# 256 x 256 direct-load tiles; at 16 pairs QKV, o and down on direct-load
-# 128 x 128 tiles and gate/up register-staged.
+# 256 x 256 direct-load tiles; at 16 pairs QKV, o and down on the small and mid M
+# tiles and gate/up register-staged.
 @pytest.mark.parametrize("bits,pairs,fused", [(4, 256, False), (8, 256, False), (4, 64, False), (8, 16, False),
                                               (4, 256, True), (8, 64, True)])
 def test_quantised_engine_equals_bf16_engine_on_dequantised_weights(dev, bits, pairs, fused):
@@ -112,6 +113,30 @@ def test_quantised_engine_equals_bf16_engine_on_dequantised_weights(dev, bits, p
         for k in oq:
             assert torch.equal(oq[k], oe[k]), (rep, k)
     assert int(oq["unmask"].sum()) > 0
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_quantised_prefill_at_every_tile_size(dev, bits):
+    """One prefix of any length runs every fused epilogue (QKV, SwiGLU, residual) at that many rows: on each tile
+    of the small and mid M kernel, both sides of its limit and with a partial last tile.  The second layer's keys
+    and values, which see the first layer's outputs at every row, and the SOS hidden equal the bf16 engine's."""
+    lens = (1, 15, 17, 32, 33, 64, 65, 100, 127, 129, 200, 257, 321, 400, 513, 641, 1000, 1025, 1281, 1500, 2049, 2300)
+    model_q = make_t3(n_layers=2, seed=80, norm_jitter=True, device=dev)
+    model_e = make_t3(n_layers=2, seed=80, norm_jitter=True, device=dev)
+    dequantize_model_(model_e, bits)
+    engines = [HipEngine(m, max(lens), torch.bfloat16, batch_size=1, page_table_seed=1, quant_bits=b)
+               for m, b in ((model_q, bits), (model_e, 0))]
+    g = torch.Generator().manual_seed(bits)
+    for n in lens:
+        prefix = torch.randn(n, D, generator=g).to(torch.bfloat16).to(dev)
+        got = []
+        for eng in engines:
+            out = [eng.prefix_forward([prefix])]
+            for pool in eng._kv.pools:
+                out += kernels.kv_gather(pool, eng._kv.table[0], n)
+            got.append(out)
+        for i, (q, e) in enumerate(zip(*got)):
+            assert torch.isfinite(q.float()).all() and torch.equal(q, e), (n, i)
 
 
 def test_thirty_layer_step_on_4bit_weights_against_the_oracle(dev):
