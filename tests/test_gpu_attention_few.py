@@ -157,3 +157,21 @@ def test_empty_rows(dev, rows, empty_item):
         outs.append(out)
     assert not outs[1][0].any() and not outs[1][-1].any()
     assert torch.equal(outs[0][1:-1], outs[1][1:-1])
+
+
+def test_long_work_list(dev):
+    """A caller's own list of 300,000 items, all but one empty and bound for no slot: one row's ring launch would hold
+    more threads than a grid can (300,000 x 48 heads x 320 > 2^32), the paged kernel's does not."""
+    H, bl, n = 48, 64, 100
+    g = torch.Generator(device=dev).manual_seed(1)
+    table = torch.randperm(8, generator=g, device=dev).to(torch.int32).view(1, 8)
+    pool = torch.randn(8, 2, H, 1024, generator=g, device=dev).to(BF)
+    q = torch.randn(1, bl, H, 64, generator=g, device=dev).to(BF)
+    outs = []
+    for items in (1, 300_000):
+        plan = AttnPlan([n], bl, H, torch.device(dev))
+        plan.work = torch.cat([plan.work, torch.tensor([[0, 0, 0, 7]], dtype=torch.int32, device=dev).repeat(items - 1, 1)])
+        out = torch.full_like(q, float("nan"))
+        plan.run(q, pool, table, out, 0.125)
+        outs.append(out)
+    assert torch.equal(*outs)

@@ -650,6 +650,9 @@ extern "C" int yapd_attn_plan(const int32_t* kv_len, int rows, int target_items,
 namespace yapd {
 namespace {
 
+// Workgroups of at most 320 threads that a launch of fewer than 2^32 threads holds, with room.
+constexpr int64_t kRingGrid = 1 << 22;
+
 // The ring kernel while its head-wide workgroups and their waves leave room on
 // the chip: 96 rows of 16 heads, 64 with three tiles, 24 with four (or, where no
 // more than 48 rows' worth of work items are asked for, three workgroups per CU of
@@ -669,7 +672,7 @@ namespace {
 template <int NQT>
 void launch_paged(const AttnParams& P, int n_work, hipStream_t st) {
   const int64_t row_heads = static_cast<int64_t>(P.rows) * P.H, wgs = static_cast<int64_t>(n_work) * P.H;
-  if ((row_heads <= (NQT == 4 ? 384 : NQT == 3 ? 1024 : 1536) || (NQT == 4 && wgs <= 768)) && wgs <= INT32_MAX) {
+  if ((row_heads <= (NQT == 4 ? 384 : NQT == 3 ? 1024 : 1536) || (NQT == 4 && wgs <= 768)) && wgs <= kRingGrid) {
     const int lds = row_heads <= 1024 ? 40 * 1024 : kRing * kRingStage;
     hipLaunchKernelGGL(attn_ring_kernel<NQT>, dim3(n_work * P.H), dim3(64 * (NQT + 1)), lds, st, P);
   } else {
