@@ -63,7 +63,9 @@ int yapd_abi_version(void);
  * Outputs [n_pairs, bl]: sampled (int64), pmi (fp32), unmask (u8), xt_out
  * (int64); per pair: n_mask_after (int32), hit_eos (u8).  1 <= bl <= 64, 1 <= K <= 64.
  * One launch: a workgroup per pair, one wave per position, then the pair's
- * pmi and decision by one wave (lane = position) from LDS.
+ * pmi and decision by one wave (lane = position) from LDS.  Up to 128 pairs of
+ * more than 8 positions: two launches, positions first, then a wave per pair.
+ * sampled_out and xt_out may be xt_in.
  * ------------------------------------------------------------------------ */
 
 int yapd_score_cfg_pmi_unmask(

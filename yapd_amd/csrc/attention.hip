@@ -654,10 +654,9 @@ namespace {
 constexpr int64_t kRingGrid = 1 << 22;
 
 // The ring kernel while its head-wide workgroups and their waves leave room on
-// the chip: 96 rows of 16 heads, 64 with three tiles, 24 with four (or, where no
-// more than 48 rows' worth of work items are asked for, three workgroups per CU of
-// their five waves each); more rows keep enough page streams in flight with four
-// heads to a workgroup.  Up to 64 rows it asks for LDS that holds it to four
+// the chip: 96 rows of 16 heads, 64 with three tiles, with four, whose workgroups
+// are five waves, 24 rows or 48 work items (three workgroups per CU); more rows keep
+// enough page streams in flight with four heads to a workgroup.  Up to 64 rows it asks for LDS that holds it to four
 // workgroups per CU, as many as unsplit rows need: on long rows six are more
 // scattered page streams at once (64 rows x 16 on 2000-2048 keys 98.8 against 94.6
 // us).  Measured (us per launch, paged -> ring; bit-identical): blocks of 32 on

@@ -960,7 +960,7 @@ __device__ __forceinline__ bool c_vec4(const GemmParams& p) {
 
 // This lane's residual values (kEpiResidual), requested before the main loop:
 // behind it they would cost a memory latency each, as every store to C could
-// alias the next load (down, M = 1630: 25.1 -> 22.4 us).
+// alias the next load (down, M = 1630: 25.1 -> 24.2 us).
 template <class T>
 __device__ __forceinline__ void sk_residual(const GemmParams& p, int m0, int bx, int wm, int wn, int tok, int sub,
                                             u32x2_t (&res)[T::TM][T::TN]) {
@@ -2348,13 +2348,12 @@ int launch_gemm(GemmParams p, hipStream_t st) {
     }
   }
   // Small and mid M: the smallest tile of gemm_sk_kernel whose grid is at most
-  // one workgroup per CU (two for 16 x 16, of 64 KB of LDS each).  Measured (us,
-  // one graph of 24 calls over 24 weights; one-wave 64 x 64 and three-stage
-  // 128 x 128 tiles before -> now, bit-identical): o M = 64 12.0 -> 3.5, 256
-  // 12.0 -> 4.9, 1000 12.7 -> 7.3, 1900 13.8 -> 9.5, 4096 14.5 -> 13.9; down
-  // M = 64 33.8 -> 6.0, 256 33.4 -> 9.0, 1000 34.5 -> 16.7, 1900 37.8 -> 23.3,
-  // 4096 47.0 -> 38.5; QKV M = 64 12.9 -> 5.1, 512 14.7 -> 10.3; gate/up M = 64
-  // 11.3 -> 6.6, 512 14.5 -> 13.1.  The next larger tile at the same M is slower
+  // one workgroup per CU.  Measured (us, one graph of 24 calls over 24 weights, with
+  // their epilogues; one-wave 64 x 64 and three-stage 128 x 128 tiles before -> now,
+  // bit-identical): o M = 64 12.5 -> 3.6, 256 12.5 -> 4.3, 1000 13.0 -> 6.4, 1900
+  // 14.3 -> 10.0; down M = 64 35.0 -> 6.0, 256 35.2 -> 7.8, 1000 35.9 -> 15.8, 1900
+  // 38.3 -> 23.5, 4096 44.1 -> 38.5; QKV M = 64 13.0 -> 5.0, 512 15.0 -> 11.2; gate/up
+  // M = 64 12.1 -> 6.8, 512 14.3 -> 13.5.  The next larger tile at the same M is slower
   // by 5 - 50 % (fewer CUs load), the next smaller one by its second round.
   // Tiles in row bands per XCD where A is the larger operand (down M = 4096
   // 45.1 -> 38.5 us), else column bands.
@@ -2391,14 +2390,17 @@ int launch_gemm(GemmParams p, hipStream_t st) {
   } else {
     const int64_t small_tiles = static_cast<int64_t>((p.M + 127) / 128) * ((p.N + 127) / 128);
     // Quantised W: the same rule on gemm_skq_kernel's tiles.  Measured (us, one
-    // graph of 24 calls over 12 weights, 4 bits; 128 x 128 tiles of
-    // gemm_dlq_kernel before -> now, bit-identical): QKV M = 64 12.9 -> 5.9, 400
-    // 14.1 -> 10.8; o M = 64 12.7 -> 4.3, 900 14.8 -> 8.1; gate/up M = 64 14.1 ->
-    // 6.9; down M = 64 47.3 -> 8.1, 400 48.9 -> 16.0, 900 52.6 -> 21.1, 1900 69.7
-    // -> 27.3, 4095 69.7 -> 45.9 (8 bits within 3 %).  16 waves in the larger
-    // tiles: every wave dequantises, and few compute waves of 64 x 32 read the
-    // fewest fragments from LDS (128 x 64 tiles, down M = 1900: 8 waves of 32 x 32
-    // 32.4, 4 of 64 x 32 27.3).
+    // graph of 24 calls over 12 weights, plain store; 128 x 128 tiles of
+    // gemm_dlq_kernel before -> now, bit-identical), 4 bits: QKV M = 64 13.3 -> 5.8,
+    // 400 14.1 -> 10.3; o M = 64 12.8 -> 4.3, 900 14.6 -> 8.0; gate/up M = 64 14.0 ->
+    // 7.0; down M = 64 45.8 -> 8.0, 400 47.9 -> 15.9, 900 53.6 -> 20.8, 1900 69.8 ->
+    // 27.5, 4095 69.8 -> 46.1.  8 bits: QKV 13.9 -> 6.0, 14.3 -> 10.8; o 12.4 -> 4.2,
+    // 15.3 -> 8.4; gate/up 14.1 -> 7.3; down 50.9 -> 7.9, 55.6 -> 15.9, 63.4 -> 21.6,
+    // 67.8 -> 44.5, 69.0 -> 46.7: with K = 4096 the 128 x 64 tile's ring of 8-bit codes
+    // leaves no room for the scales (172 KB of 160), and its rows, 1025 to 2048, run on
+    // the 128 x 128 tile, half of the CUs.  16 waves in the larger tiles: every wave
+    // dequantises, and few compute waves of 64 x 32 read the fewest fragments from LDS
+    // (128 x 64 tiles, down M = 1900: 8 waves of 32 x 32 32.4, 4 of 64 x 32 27.3).
     p.xcd_band = p.M > p.N ? 1 : 0;
     if constexpr (EPI == kEpiStore || EPI == kEpiResidual) {
       if (skq_fits<Skq16<BQ>>(p, cus)) return launch_skq<Skq16<BQ>, EPI, BQ>(p, st);
@@ -2574,7 +2576,8 @@ int rmsnorm_launch(const void* delta, void* residual, const void* x, const void*
   // Few rows: one latency chain per row, on a CU of its own while there are few
   // (behind the GEMM that wrote x, us, two rows a wave -> this: M = 64 3.26 -> 2.46,
   // 256 3.73 -> 3.00; four waves of one row each 64 2.76, 600 5.08 -> 4.44, 1000 6.35
-  // -> 5.83, 3000 8.34 -> 7.45, 4096 9.23 -> 9.87).
+  // -> 5.83, 3000 8.34 -> 7.45, 4096 9.23 -> 9.87, 8192 8.72 -> 8.08, 16384 11.66 ->
+  // 11.80: above 3072 neither leads throughout, and two rows a wave is kept).
   if (M <= 512) {
     hipLaunchKernelGGL(rmsnorm_kernel<1>, dim3(M), dim3(64), 0, st, p);
   } else if (M <= 3072) {

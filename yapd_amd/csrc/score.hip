@@ -553,7 +553,7 @@ __global__ __launch_bounds__(64) void score_decide_kernel(const ScoreParams P) {
 }
 
 // score_pair_kernel leaves the CUs without a pair idle and one wave takes up to
-// four positions in turn; two launches pay while pairs fill at most half of the
+// four positions in turn; two launches pay while pairs fill at most half of the 256
 // CUs and a pair has more positions than half of its waves.  Measured (us, with a
 // null row, pair kernel -> two launches): blocks of 32, 1 pair 30.7 -> 11.1, 32
 // 32.5 -> 14.4, 128 40.2 -> 32.9, 192 44.7 -> 45.2; of 16, 5 17.9 -> 11.5, 128
