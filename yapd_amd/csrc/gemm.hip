@@ -834,8 +834,8 @@ __global__ __launch_bounds__(T::THREADS) void gemm_dl_kernel(const GemmParams p)
   int stage = 0;
   for (int kt = 0; kt < kt_n; ++kt) {
     const bool more = kt + 1 < kt_n;
-    const int next = stage + 1 == NS ? 0 : stage + 1;
-    if (kt + NS - 1 < kt_n) issue(kt + NS - 1, stage == 0 ? NS - 1 : stage - 1);
+    const int next = NS == 2 ? stage ^ 1 : stage + 1 == NS ? 0 : stage + 1;
+    if (kt + NS - 1 < kt_n) issue(kt + NS - 1, NS == 2 ? next : stage == 0 ? NS - 1 : stage - 1);
 #pragma unroll
     for (int ks = 0; ks + 1 < KS; ++ks) {
       read_frags(stage, ks + 1, (ks + 1) & 1);
