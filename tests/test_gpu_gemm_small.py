@@ -182,3 +182,25 @@ def test_few_columns_of_many_rows(dev, N):
     ref = A.double() @ W.double().T
     mag = A.double().abs() @ W.double().abs().T
     assert ((C.double() - ref).abs() <= ref.abs() * 2.0 ** -8 + mag * K * 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("epi", ["store", "residual", "swiglu"])
+@pytest.mark.parametrize("off,pitch", [(0, 1), (1, 0), (2, 2), (4, 4)])
+def test_output_rows_anywhere(dev, epi, off, pitch):
+    """C from any element on and with any row pitch, on each tile: the values of a packed call, and nothing beside
+    them."""
+    N, K = 256, 512
+    for M in (3, 100, 257, 1000, 2049, 4100, 9000):
+        A, W = rnd(M, K, std=0.5, seed=31), rnd(2 * N if epi == "swiglu" else N, K, std=0.05, seed=32)
+        R = rnd(M, N, seed=33)
+        f = {"store": kernels.gemm_bf16, "residual": kernels.gemm_bf16_residual, "swiglu": kernels.gemm_swiglu}[epi]
+        C = R.clone()
+        f(A, W, C)
+        ld = N + pitch + off
+        wide = torch.full((M * ld + 8,), 7.0, dtype=BF, device=dev)
+        out = torch.as_strided(wide, (M, N), (ld, 1), off)
+        out.copy_(R)
+        f(A, W, out)
+        assert torch.equal(out, C), M
+        out.fill_(7.0)
+        assert (wide == 7.0).all(), M
